@@ -24,7 +24,7 @@
 //     (5,7) to match the packed-quant extraction.
 //   * activations go through LDS as f16, double buffered: the next super-block's global
 //     loads are in flight while the current one runs on the matrix cores.
-#include "common.h"
+#include "matmul_common.h"
 
 namespace {
 
@@ -33,16 +33,6 @@ constexpr uint32_t TILE_MAP = 640;  // words of moe_sort's tile map before its t
 constexpr int KC = 256;        // k per LDS stage (one K-quant super-block)
 constexpr int PITCH = KC + 8;  // f16 per staged token row (16 B pad: conflict-free b128)
 
-struct MatmulPush {  // 13 words (graph.rs:27-32, graph/moe.rs:26-40)
-  uint32_t o0, o1, o2, o3, x_off, y_off, n_in, n_out, x_stride, y_stride, table_off, list_off,
-      x_div;
-};
-
-SK_DEV f16x2 splat(f16 v) {
-  f16x2 r = {v, v};
-  return r;
-}
-
 // k offset (inside the current 256-k stage) of the 8 values lane-half hh holds at step t
 template <int TYPE>
 SK_DEV uint32_t koff(int t, uint32_t hh) {
@@ -50,28 +40,6 @@ SK_DEV uint32_t koff(int t, uint32_t hh) {
   if (TYPE == 2) return 128 * (t >> 3) + 32 * ((t >> 1) & 3) + 16 * (t & 1) + 8 * hh;  // Q6_K
   return 16 * t + 8 * hh;                                                            // Q8_0
 }
-
-// Raw weight bytes of one row for one 256-k stage, held by each lane.
-template <int TYPE>
-struct WStage;
-
-template <>
-struct WStage<1> {  // Q4_K: 128 B qs + 16 B header
-  uint4 qs[8];
-  uint4 hd;
-};
-template <>
-struct WStage<2> {  // Q6_K: ql 128 B, qh 64 B, 16 scales, d
-  uint4 ql[8];
-  uint4 qh[4];
-  uint4 sc;
-  uint32_t d;
-};
-template <>
-struct WStage<0> {  // Q8_0: 8 blocks of 32 quants + 8 scales
-  uint4 q[16];
-  uint32_t d[8];
-};
 
 template <int TYPE>
 SK_DEV void load_stage(WStage<TYPE> &s, const uint4 *w, const uint16_t *wd, const MatmulPush &p,
@@ -182,34 +150,6 @@ SK_DEV f16x8 weight_frag(const WStage<TYPE> &s, int t, uint32_t hh, f16x2 scale,
     (void)m1;
     f16x8 r = {w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
     return r;
-  }
-}
-
-// Scale (and negated min) of lane half hh at step t, as f16 pairs.  The f32 products
-// d*sc and dmin*m are the reference's d0 / min0 (quant.rs:60-61), rounded once to f16.
-template <int TYPE>
-SK_DEV void step_scale(const WStage<TYPE> &s, int t, uint32_t hh, f16x2 &scale, f16x2 &negmin) {
-  if constexpr (TYPE == 1) {
-    const uint32_t j = 2 * (t >> 2) + hh;
-    uint32_t sc, m;
-    q4k_scale_min(j, s.hd.y, s.hd.z, s.hd.w, sc, m);
-    const float d = f16_bits_to_f32(s.hd.x & 0xffffu);
-    const float dmin = f16_bits_to_f32(s.hd.x >> 16);
-    // high nibbles arrive as 16q: fold the 1/16 into the scale
-    const float sc_f = d * (float)sc * (hh ? 0.0625f : 1.0f);
-    scale = splat((f16)sc_f);
-    negmin = splat((f16)(-(dmin * (float)m)));
-  } else if constexpr (TYPE == 2) {
-    const int hf = t >> 3, g = (t >> 1) & 3;
-    const uint32_t k = 8 * hf + (t & 1) + 2 * g;
-    const uint32_t wv = k < 4 ? s.sc.x : (k < 8 ? s.sc.y : (k < 12 ? s.sc.z : s.sc.w));
-    const int sc = (int)(int8_t)((wv >> (8 * (k & 3))) & 255u);
-    const float d = f16_bits_to_f32(s.d);
-    scale = splat((f16)(d * (float)sc * (g >= 2 ? 0.0625f : 1.0f)));
-    negmin = splat((f16)0.0f);
-  } else {
-    scale = splat(__builtin_bit_cast(f16, (uint16_t)s.d[t >> 1]));
-    negmin = splat((f16)0.0f);
   }
 }
 
@@ -436,15 +376,6 @@ constexpr int KX_W = 256;           // k per activation chunk: K-quant tiles (on
 constexpr int KX_Q8 = 128;          // k per activation chunk: Q8_0 tile (register weights)
 constexpr int DL_KX = 64;           // k per activation chunk: direct-to-LDS tile
 
-// 16 B unit slot swizzle of a direct-to-LDS row (128 B rows, 8 units): distinct banks for 16
-// consecutive rows in a 256 B bank line and for 8 in a 128 B one
-SK_DEV uint32_t dl_swz(uint32_t r) { return (r & 7u) ^ ((r >> 3) & 1u); }
-typedef __attribute__((address_space(3))) void dl_lds;
-// vmcnt(N), the other counters unconstrained (gfx9 s_waitcnt encoding)
-template <int N>
-SK_DEV void dl_wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
-}
 template <int KX>
 constexpr int pitch2() { return KX + 8; }  // f16 per staged token row (16 B pad)
 
@@ -865,7 +796,6 @@ SK_DEV void lds_scales(const uint32_t *row, uint32_t hh, StageScales<TYPE> &o) {
 // y_off, n_out, y_stride); x_off, n_in and x_stride are the same for all.
 // Per-lane state of the direct-to-LDS tile: buffer resources, this lane's load offsets
 // (activation pieces, weight pieces) and its read swizzles.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Weight stage layout of the direct-to-LDS tile (byte offsets in one stage buffer; each
 // region is whole 1 KiB blocks, loaded block by block, one 16 B piece per lane):
@@ -896,34 +826,6 @@ struct DLLanes {
   uint32_t wv, lane, lrow, hh, tb, wsw, wsw4, xsw;
   uint32_t dpos0;  // Q6_K: byte offset of this lane's row's d at super-block 0
 };
-
-// Buffer resource words over [base, base + bytes) (as buf_res builds them: stride 0, raw
-// 32-bit data), for the loads below, which take it as an SGPR quad.
-SK_DEV u32x4 dl_res(const void *base, uint64_t bytes) {
-  const uint64_t a = (uint64_t)base;
-  u32x4 r = {(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, (uint32_t)(bytes < 0xffffffffull ? bytes : 0xffffffffull),
-             0x00020000u};
-  return r;
-}
-// One 16 B-per-lane buffer load into LDS: lane l's 16 B land at byte lds + 16 l (wave-
-// uniform lds, in M0); a load past the resource's end writes zeros.  Written as assembly on
-// purpose: with the compiler's own form of this load, every later LDS read waits until all
-// such loads in flight are done (the compiler cannot tell which LDS bytes they write),
-// which serialises the double buffering; here the explicit waits of dl_stage order each
-// buffer's loads before its reads, and the compiler's own waits (it does not count these
-// loads) can only wait longer than needed, never less.
-// (m0 is declared clobbered; the compiler warns that it reserves m0, which these kernels
-// use for nothing else)
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-SK_DEV void dl_load16(const u32x4 &res, uint32_t lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(lds), "v"(voff), "s"(res), "s"(soff)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-SK_DEV uint32_t lds_addr(const void *p) { return (uint32_t)(uintptr_t)(dl_lds *)p; }
 
 // Source of weight block b for this lane: byte offset (super-block 0) and bytes per
 // super-block, with rows past n_out clamped to the last row.

@@ -12,6 +12,7 @@ sym##_end:                          \
     .section .rodata
 EMBED(skyla_co_matvec, "matvec.hsaco")
 EMBED(skyla_co_matmul, "matmul.hsaco")
+EMBED(skyla_co_matmul_ring, "matmul_ring.hsaco")
 EMBED(skyla_co_moe, "moe.hsaco")
 EMBED(skyla_co_util, "util.hsaco")
 EMBED(skyla_co_attention, "attention.hsaco")

@@ -32,6 +32,7 @@
 // Code objects embedded by embed.S.
 extern "C" const unsigned char skyla_co_matvec[], skyla_co_matvec_end[];
 extern "C" const unsigned char skyla_co_matmul[], skyla_co_matmul_end[];
+extern "C" const unsigned char skyla_co_matmul_ring[], skyla_co_matmul_ring_end[];
 extern "C" const unsigned char skyla_co_moe[], skyla_co_moe_end[];
 extern "C" const unsigned char skyla_co_util[], skyla_co_util_end[];
 extern "C" const unsigned char skyla_co_attention[], skyla_co_attention_end[];
@@ -92,6 +93,7 @@ const Tactic kTactics[] = {
     {"xhalf_moe", "1", "expert-group matmuls on f32 rows take the f16 row prepass (0: the tile's own f32 staging)"},
     {"xhalf_join", "1", "a dense matmul's f16 row prepass runs in the rmsnorm or silu_mul launch that writes its "
                         "rows (0: a launch of its own)"},
+    {"ring", "1", "dense matmuls on f16 rows take the ring tiles (0: never; WR_WK_NB_DX_S: that shape, split S ways)"},
     {"dl", "1", "matmul tiles with their operands loaded straight into LDS (0: register-staged)"},
     {"merge_t", "1", "batched attention merge as one wave per (head, token) (0: 1024-thread form)"},
     {"nograph", "0", "1: recordings replay as direct launches instead of one HIP graph (kernel traces)"},
@@ -186,6 +188,23 @@ const KernelInfo *find_kernel(const char *name) {
 constexpr uint64_t kScratchTiles = 256;
 constexpr uint64_t kScratchCounters = 1024;
 
+// Shapes of the ring tile (matmul_ring.hip, matmul_ring__T_A_WR_WK_NB_DX): 32 wr rows x 32 nb
+// tokens a workgroup of wr x wk waves, its K split wk ways inside the workgroup.
+struct RingShape {
+  uint32_t wr, wk, nb, dx;
+};
+enum { kRingWide, kRingPair, kRingHalves, kRingQuarters, kRingShapes };
+constexpr RingShape kRing[kRingShapes] = {
+    {4, 1, 4, 4},  // wide: 128 rows x 128 tokens, one workgroup per CU
+    {4, 1, 4, 3},  // pair: the same with a ring of three chunks, two workgroups per CU
+    {4, 2, 2, 4},  // halves: 128 rows x 64 tokens, eight waves, K in halves
+    {1, 4, 2, 3},  // quarters: 32 rows x 64 tokens, four waves, K in quarters
+};
+struct RingFns {
+  hipFunction_t fn[kRingShapes];
+  uint32_t type;  // 0 Q8_0, 1 Q4_K, 2 Q6_K
+};
+
 struct skyla_hip_context {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -203,6 +222,7 @@ struct skyla_hip_context {
   hipFunction_t silu_mul = nullptr;        // (moe.hip): the launch it replaces
   hipFunction_t rmsnorm_half_rows = nullptr;  // rmsnorm with a dense matmul's prepass (matmul.hip)
   hipFunction_t rmsnorm = nullptr;            // (attention.hip): the launch it replaces
+  std::shared_ptr<const RingFns> ring[3][2];  // the ring tiles by weight type and ACCUM
 };
 
 struct HostFree {
@@ -258,6 +278,7 @@ struct skyla_hip_pipeline {
   hipFunction_t hxs_fn = nullptr;        // the eight-wave tile over several matrices (segments)
   hipFunction_t hxm_fn = nullptr;        // expert groups (MOE = 1) on x_half_rows's f16 rows
   hipFunction_t hxms_fn = nullptr;       // and over several matrices on the same rows (segments)
+  std::shared_ptr<const RingFns> ring;   // dense matmul on f16 rows: the ring tiles
   uint32_t split_threads = 0;
   hipFunction_t tok_fn = nullptr;        // batched form: a tok_per_wg x tok_per_wg_y block of
   uint32_t tok_per_wg = 0;               // grid.x and grid.y per workgroup
@@ -282,6 +303,7 @@ struct Command {
   uint32_t split_threads = 0;
   hipFunction_t hx_fn = nullptr, hx4_fn = nullptr, hx4b_fn = nullptr, hxs_fn = nullptr, hxm_fn = nullptr,
                 hxms_fn = nullptr;
+  std::shared_ptr<const RingFns> ring;
   hipFunction_t tok_fn = nullptr;
   uint32_t tok_per_wg = 0, tok_per_wg_y = 0, tok_threads = 0;
   std::string name;                 // the pipeline's shader name
@@ -568,9 +590,55 @@ Launch x_half_prepass(skyla_hip_context *ctx, const Command &a, uint64_t h_bytes
 // same kernel, bindings and token grid, and the same activation rows (x_off, n_in,
 // x_stride); dispatches with no barrier between them are independent.
 bool fusable_matmul(const Command &a, const Command &c) {
-  return c.kind == Command::Dispatch && c.hx_fn == a.hx_fn && c.hxs_fn == a.hxs_fn && !c.segmented &&
-         c.push.size() == 13 && c.bufs == a.bufs && c.groups[1] == 1 && c.groups[2] == a.groups[2] &&
+  return c.kind == Command::Dispatch && c.fn == a.fn && c.hx_fn == a.hx_fn && c.hxs_fn == a.hxs_fn &&
+         c.ring == a.ring && !c.segmented && c.push.size() == 13 && c.bufs == a.bufs && c.groups[1] == 1 && c.groups[2] == a.groups[2] &&
          c.push[4] == a.push[4] && c.push[6] == a.push[6] && c.push[8] == a.push[8];
+}
+
+// Can dense matmul a run on the ring tiles?  Both weight bindings must be one buffer (the tile
+// reads it through one resource), the f16 rows and a tile's output rows must stay within the
+// 2 GiB its 32-bit offsets reach.
+bool ring_fits(const Command &a) {
+  if (!a.ring || a.bufs[0] != a.bufs[1]) return false;
+  const uint64_t rows = (uint64_t)a.groups[2] * 128, n_in = a.push[6];
+  return a.groups[0] == (a.push[7] + 127) / 128 && n_in % (a.ring->type == 0 ? 32 : 256) == 0 && rows * n_in * 2 + rows * 4 + 256 < 0x7fffffffull &&
+         (a.push[9] + (uint64_t)a.push[7]) * 128 * 4 < 0x7fffffffull;
+}
+
+// The ring shape and K split of a launch over `tiles` tiles of 128 rows x 128 tokens (rows32
+// blocks of 32 rows in all, n_tok tokens), from sweeps on MI355X (us, weights from HBM, the
+// eight-wave tile before it in parentheses):
+//   more than 256 tiles      two workgroups per CU: Q4_K 12288 x 4096, M = 512 65 (wide 71, 75)
+//   from 96                  wide: 24576 x 4096 at M = 128 37 (60); with 97..128 tiles half the
+//                            CUs would idle, so K in two splits: 4096 x 4096 at M = 512 31 (37),
+//                            Q6_K 4096 x 12288 83 (103)
+//   fewer, short K           quarters while rows32 x token tiles x super-blocks <= 4096: 4096 x
+//                            4096 at M = 128 14.2 (26; halves split two ways 16.4), Q8_0 3072 x
+//                            1024 6.8 (43), 1024 x 3072 11.3 (126; wide 28)
+//   fewer, else              halves, split over 256 workgroups: 6144 x 4096 18.4 (25; quarters
+//                            24.9), 4096 x 12288 Q4_K 28.7 (34; quarters 36), Q6_K 35.6 (40)
+// K quarters, halves and splits keep split_stages super-blocks each (Q8_0: one 256-value
+// stage); shorter rows, and every row with the splitk tactic off, are summed whole.
+int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split) {
+  const uint32_t n_stage = (a.push[6] + 255) / 256;
+  const uint32_t ways = !a.split_fn && a.ring->type != 0 ? 1u : n_stage / (a.ring->type == 0 ? 1u : split_stages());
+  RingShape f{};
+  if (std::sscanf(tactic("ring").c_str(), "%u_%u_%u_%u_%u", &f.wr, &f.wk, &f.nb, &f.dx, split) == 5)
+    for (int i = 0; i < kRingShapes; i++)
+      if (kRing[i].wr == f.wr && kRing[i].wk == f.wk && kRing[i].nb == f.nb && kRing[i].dx == f.dx) {
+        *split = std::max(1u, std::min(std::min(*split, n_stage), 8u));
+        return i;
+      }
+  *split = 1;
+  if (tiles > 256) return kRingPair;
+  if (tiles >= 96 || ways < 2) {
+    if (tiles > 96 && tiles <= 128 && ways >= 2) *split = 2;
+    return kRingWide;
+  }
+  const uint64_t tok64 = (uint64_t)a.groups[2] * 2;
+  if (ways >= 4 && rows32 * tok64 * n_stage <= 4096) return kRingQuarters;
+  *split = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({256 / (tiles * 2), ways / 2, 8}));
+  return kRingHalves;
 }
 
 // The launch list of a recording.  Barriers need no command of their own: launches on one
@@ -699,8 +767,10 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
       i += n_run;
       continue;
     }
-    if (xhalf && a.hx_fn && !a.segmented && a.push.size() == 13 && a.bufs.size() == 5 && a.groups[1] == 1 &&
-        a.push[6] % 256 == 0 && a.push[6] <= 12288 && a.push[4] % 4 == 0 && a.push[8] % 4 == 0) {
+    const bool dense = xhalf && !a.segmented && a.name == "matmul" && a.push.size() == 13 && a.bufs.size() == 5 &&
+                       a.groups[1] == 1 && a.push[6] <= 12288 && a.push[4] % 4 == 0 && a.push[8] % 4 == 0;
+    const bool ring = dense && xh == "1" && ring_fits(a);
+    if (ring || (dense && a.hx_fn && a.push[6] % 256 == 0)) {
       const uint32_t rows = a.groups[2] * 128;
       const uint64_t h_off = ((uint64_t)rows * 4 + 255) & ~(uint64_t)255;
       const std::vector<uint32_t> key = {(uint32_t)((uintptr_t)a.bufs[2] >> 32), (uint32_t)(uintptr_t)a.bufs[2],
@@ -750,6 +820,52 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
       uint32_t n_run = 1;
       uint64_t row_tiles = a.groups[0];
       const long seg_big = std::atol(tactic("seg_big").c_str());
+      if (ring) {
+        // any run of matrices on these rows (seg_big 0: while it has at most 128 tiles)
+        while (fuse && n_run < kMaxSeg && i + n_run < cmds.size() && fusable_matmul(a, cmds[i + n_run]) &&
+               ring_fits(cmds[i + n_run]) &&
+               (seg_big > 0 || (row_tiles + cmds[i + n_run].groups[0]) * a.groups[2] <= 128)) {
+          row_tiles += cmds[i + n_run].groups[0];
+          n_run++;
+        }
+        uint64_t rows32 = 0;
+        for (uint32_t q = 0; q < n_run; q++) rows32 += (cmds[i + q].push[7] + 31) / 32;
+        uint32_t S = 1;
+        const int f = ring_rule(a, row_tiles * a.groups[2], rows32, &S);
+        const RingShape &r = kRing[f];
+        Launch l;
+        l.fn = a.ring->fn[f];
+        l.threads = 64 * r.wr * r.wk;
+        l.bufs = a.bufs;
+        const size_t w = 13;
+        l.args.assign(1 + kMaxSeg + kMaxSeg * w, 0u);
+        l.args[0] = n_run;
+        uint32_t start = 0;
+        for (uint32_t q = 0; q < kMaxSeg; q++) {
+          l.args[1 + q] = q < n_run ? start : 0xffffffffu;
+          if (q < n_run) {
+            const Command &c = cmds[i + q];
+            uint32_t *dst = l.args.data() + 1 + kMaxSeg + q * w;
+            std::copy(c.push.begin(), c.push.end(), dst);
+            dst[4] = (uint32_t)(h_off / 2);  // f16 units
+            dst[8] = a.push[6];
+            start += (c.push[7] + 32 * r.wr - 1) / (32 * r.wr);
+          }
+        }
+        l.groups[0] = start;
+        l.groups[1] = 1;
+        l.groups[2] = a.groups[2] * (4 / r.nb) * S;
+        l.split = S;
+        if (S > 1) {
+          l.n_cnt = start * a.groups[2] * (4 / r.nb);
+          l.ws_bytes = (uint64_t)l.n_cnt * S * r.wr * r.wk * std::max(1u, r.nb / r.wk) * 4096;
+        }
+        l.xh_buf = 2;
+        l.xh_bytes = out.back().xh_bytes;
+        out.push_back(std::move(l));
+        i += n_run;
+        continue;
+      }
       const uint64_t max_tiles = seg_big > 0 ? 256 : 128;
       if (fuse && a.hxs_fn && a.split_fn) {
         while (n_run < kMaxSeg && i + n_run < cmds.size() && fusable_matmul(a, cmds[i + n_run]) &&
@@ -955,6 +1071,7 @@ Command dispatch_command(const skyla_hip_pipeline *p, const std::vector<void *> 
   c.hx4_fn = p->hx4_fn;
   c.hx4b_fn = p->hx4b_fn;
   c.hxs_fn = p->hxs_fn;
+  c.ring = p->ring;
   c.split_threads = p->split_threads;
   c.tok_fn = p->tok_fn;
   c.tok_per_wg = p->tok_per_wg;
@@ -1207,8 +1324,8 @@ int skyla_hip_context_new(int device, skyla_hip_context **out) {
   ctx->name += std::string(" (") + prop.gcnArchName + ", " + std::to_string(prop.multiProcessorCount) + " CUs)";
   ctx->warp = (uint32_t)prop.warpSize;
   HIP_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
-  const unsigned char *images[] = {skyla_co_matvec, skyla_co_matmul, skyla_co_moe, skyla_co_util,
-                                   skyla_co_attention};
+  const unsigned char *images[] = {skyla_co_matvec, skyla_co_matmul, skyla_co_matmul_ring, skyla_co_moe,
+                                   skyla_co_util, skyla_co_attention};
   for (const unsigned char *img : images) {
     hipModule_t m = nullptr;
     hipError_t le = hipModuleLoadData(&m, img);
@@ -1245,6 +1362,21 @@ int skyla_hip_context_new(int device, skyla_hip_context **out) {
   ctx->silu_mul = find_function(ctx.get(), "silu_mul");
   ctx->rmsnorm_half_rows = find_function(ctx.get(), "rmsnorm_half_rows");
   ctx->rmsnorm = find_function(ctx.get(), "rmsnorm");
+  for (uint32_t t = 0; t < 3; t++)
+    for (uint32_t acc = 0; acc < 2; acc++) {
+      auto ring = std::make_shared<RingFns>();
+      ring->type = t;
+      bool all = true;
+      for (int i = 0; i < kRingShapes; i++) {
+        const RingShape &r = kRing[i];
+        const std::string sym = "matmul_ring__" + std::to_string(t) + "_" + std::to_string(acc) + "_" +
+                                std::to_string(r.wr) + "_" + std::to_string(r.wk) + "_" + std::to_string(r.nb) + "_" +
+                                std::to_string(r.dx);
+        ring->fn[i] = find_function(ctx.get(), sym);
+        all &= ring->fn[i] != nullptr;
+      }
+      if (all) ctx->ring[t][acc] = ring;
+    }
   if (prop.multiProcessorCount > 0) ctx->n_cu = (uint32_t)prop.multiProcessorCount;
   *out = ctx.release();
   return SKYLA_HIP_OK;
@@ -1454,8 +1586,8 @@ int skyla_hip_pipeline_new(skyla_hip_context *ctx, const char *name, uint32_t n_
       p->split_fn = find_function(ctx, ssym);
       p->split_threads = 512;
     }
-    // f32 inputs: the tile on x_half_rows's f16 rows (build_launches inserts the prepass),
-    // by default the forms whose operands go straight into LDS (eight waves: x8d, x8ds; four
+    // f32 inputs: the 128 x 128 tile on x_half_rows's f16 rows (build_launches inserts the
+    // prepass) where the ring tiles do not fit or are off, by default the forms whose operands go straight into LDS (eight waves: x8d, x8ds; four
     // waves, Q4_K only: x4d, x4db); the dl tactic 0 keeps the register-staged tiles.
     if (!(n_spec == 4 && spec[3])) {
       const bool dl = tactic_on("dl");
@@ -1468,6 +1600,10 @@ int skyla_hip_pipeline_new(skyla_hip_context *ctx, const char *name, uint32_t n_
       p->split_threads = 512;
     }
   }
+  // the ring tiles of a dense matmul on f32 inputs (with the dl tactic 0: never)
+  if (std::strcmp(name, "matmul") == 0 && n_spec >= 3 && spec[0] <= 2 && spec[2] == 0 && !(n_spec == 4 && spec[3]) &&
+      tactic_on("ring") && tactic_on("dl"))
+    p->ring = ctx->ring[spec[0]][spec[1] & 1];
   // expert-group K-quant matmul (MOE = 1) on f32 inputs: the same tile on x_half_rows's f16
   // rows (build_launches inserts the prepass of the launch's input rows)
   if (std::strcmp(name, "matmul") == 0 && n_spec >= 3 && (spec[0] == 1 || spec[0] == 2) && spec[2] == 1 &&
