@@ -1129,6 +1129,111 @@ SK_DEV void matvec_q8_0_body(const uint4 *__restrict__ w, const uint16_t *__rest
   store_rows<ACCUM, ROWS, LPR>(y, y_off, first, p.n_out, lane, acc, yold);
 }
 
+// ---------------------------------------------------------------------------------------
+// Q8_0 rows of at most 4096 values without staging (matvec_q8_0_ks).  KW waves split a row into
+// runs of 1024 values: lane l of wave k holds the 16 activations of unit 64 k + l in registers
+// (and their sum), loaded once, and takes that unit of each of the wave's R rows; every load of
+// the workgroup is issued at entry.  A row's lanes are summed with DPP alone.  With one wave per
+// row there is no barrier (RW such waves a workgroup); with several their sums meet in LDS once.
+// What bounds these launches (Qwen3-0.6B: 1 to 7 MB) is the chain from launch to store:
+// activations staged in LDS put a round trip through it, a barrier and the LDS reads of every
+// step on that chain.  us a launch (kernel trace), LDS-staged -> this form: q+k+v with the norm
+// 4.80 -> 3.84, o 4.16 -> 3.24, gate+up with the norm 5.60 -> 4.60, down with the SiLU 5.76 ->
+// 4.24; six layers' plain products 110.7 -> 87.5 a pass, a token 798 -> 675.
+// MODE 1 / 2: the SiLU and RMSNorm forms (fuse4); every wave holds its run of the vector, so the
+// sum of squares of the row is the sum of its waves'.
+// ---------------------------------------------------------------------------------------
+SK_DEV float wave_total(float v) {  // the sum over 64 lanes, in lanes 48..63
+  v += dpp_f<0xb1>(v);   // as lane_sum: the sum of each 16
+  v += dpp_f<0x4e>(v);
+  v += dpp_f<0x141>(v);
+  v += dpp_f<0x140>(v);
+  // row_bcast:15 into rows 1 and 3, then row_bcast:31 into rows 2 and 3
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false));
+  return v;
+}
+constexpr int q8ks_row_waves(int kw) { return kw == 1 ? 4 : kw == 2 ? 2 : 1; }
+
+template <int ACCUM, int KW, int R, int MODE = 0, typename P = MatvecPush2>
+SK_DEV void matvec_q8_0_ks_body(const uint4 *__restrict__ w, const uint16_t *__restrict__ wd, const float *x,
+                                float *y, const P &p, uint32_t bx) {
+  constexpr int RW = q8ks_row_waves(KW);
+  __shared__ float part[KW > 1 ? KW : 1][KW > 1 ? RW * R + RW : 1];
+  const uint32_t tid = threadIdx.x, l = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t wk = wv % KW, rw = wv / KW;
+  const uint32_t row0 = (bx * RW + rw) * R;
+  const uint32_t chunks = p.n_in >> 4, blocks = p.n_in >> 5;
+  const uint32_t u = wk * 64 + l, uc = min(u, chunks - 1);
+  const bool live = u < chunks;
+  const uint32_t SG = opaque_mask(0x80808080u);
+
+  const float *xv = x + p.x_off + 16 * uc;
+  float4 xk[4], ak[MODE ? 4 : 1];
+#pragma unroll
+  for (int k = 0; k < 4; k++) xk[k] = *(const float4 *)(xv + 4 * k);
+  if constexpr (MODE != 0) {
+    const float *av = x + p.aux_off + 16 * uc;
+#pragma unroll
+    for (int k = 0; k < 4; k++) ak[k] = *(const float4 *)(av + 4 * k);
+  }
+  uint4 q[R];
+  uint32_t d[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const uint32_t row = min(row0 + r, p.n_out - 1);
+    q[r] = load_nt(w + p.o0 + row * chunks + uc);
+    d[r] = load_nt(wd + p.o1 + row * blocks + (uc >> 1));
+  }
+  // lane 48 + r of a row's first wave finishes row r: its old output is read now
+  const uint32_t lr = l - 48;
+  const bool store = wk == 0 && lr < (uint32_t)R && row0 + lr < p.n_out;
+  float yold = 0.0f;
+  if constexpr (ACCUM)
+    if (store) yold = y[p.y_off + row0 + lr];
+
+  float ss = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    if constexpr (MODE != 0) xk[k] = fuse4<MODE>(xk[k], ak[k], ss);
+    if (!live) xk[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if constexpr (MODE == 2) ss = wave_total(live ? ss : 0.0f);
+  const float bias = -128.0f * ((sum4(xk[0]) + sum4(xk[1])) + (sum4(xk[2]) + sum4(xk[3])));
+  float mine = 0.0f;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    float s = bias;
+    s = fma_bytes(q[r].x ^ SG, xk[0], s);
+    s = fma_bytes(q[r].y ^ SG, xk[1], s);
+    s = fma_bytes(q[r].z ^ SG, xk[2], s);
+    s = fma_bytes(q[r].w ^ SG, xk[3], s);
+    const float t = wave_total(live ? f16_bits_to_f32(d[r]) * s : 0.0f);
+    if (lr == (uint32_t)r) mine = t;
+  }
+  if constexpr (KW > 1) {
+    if (lr < (uint32_t)R) part[wk][rw * R + lr] = mine;
+    if (MODE == 2 && lr == 0) part[wk][RW * R + rw] = ss;
+    __syncthreads();
+    if (!store) return;
+    mine = part[0][rw * R + lr];
+#pragma unroll
+    for (int k = 1; k < KW; k++) mine += part[k][rw * R + lr];
+    if constexpr (MODE == 2) {
+      ss = part[0][RW * R + rw];
+#pragma unroll
+      for (int k = 1; k < KW; k++) ss += part[k][RW * R + rw];
+    }
+  }
+  if constexpr (MODE == 2) mine *= 1.0f / sqrtf(ss / (float)p.n_in + p.eps);
+  if (store) {
+    if (ACCUM)
+      y[p.y_off + row0 + lr] = yold + mine;
+    else
+      y[p.y_off + row0 + lr] = mine;
+  }
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------------------
@@ -1369,3 +1474,23 @@ extern "C" __global__ __launch_bounds__(256) void matvec_q4k_dcomb__8(
   (void)x;  // the arena is bound as x, y and ids; y is its writable view
   matvec_q4k_dcomb_body<8>(w, y, ids, m.p[0], blockIdx.x);
 }
+
+// Q8_0 rows of at most 4096 values, KW runs of 1024 a row, R rows a wave (matvec_q8_0_ks_body)
+#define MV_Q8_0_KS(NAME, PUSH, A, KW, R, MODE)                                                          \
+  extern "C" __global__ __launch_bounds__(64 * KW * q8ks_row_waves(KW)) void NAME##__##A##_##KW##_##R( \
+      const uint4 *w, const uint16_t *wd, const float *x, float *y, const uint32_t *ids,                \
+      Segments<PUSH> m) {                                                                               \
+    const uint32_t s = segment_of(m, blockIdx.x);                                                       \
+    (void)ids;                                                                                          \
+    matvec_q8_0_ks_body<A, KW, R, MODE>(w, wd, x, y, segment_push(m, s), blockIdx.x - m.start[s]);      \
+  }
+#define MV_Q8_0_KS_FORMS(KW, R)                                   \
+  MV_Q8_0_KS(matvec_q8_0_ks, MatvecPush2, 0, KW, R, 0)            \
+  MV_Q8_0_KS(matvec_q8_0_ks, MatvecPush2, 1, KW, R, 0)            \
+  MV_Q8_0_KS(matvec_q8_0_norm_ks, MatvecPush2F, 0, KW, R, 2)      \
+  MV_Q8_0_KS(matvec_q8_0_silu_ks, MatvecPush2F, 1, KW, R, 1)
+#define MV_Q8_0_KS_ROWS(KW) MV_Q8_0_KS_FORMS(KW, 2) MV_Q8_0_KS_FORMS(KW, 4) MV_Q8_0_KS_FORMS(KW, 8)
+MV_Q8_0_KS_ROWS(1)
+MV_Q8_0_KS_ROWS(2)
+MV_Q8_0_KS_ROWS(3)
+MV_Q8_0_KS_ROWS(4)

@@ -78,6 +78,8 @@ const Tactic kTactics[] = {
                            "(empty: the engine's)"},
     {"q8_big", "4_1_16", "W_R_L: dense Q8_0 launches of 65536 rows or more (an output head) on that variant "
                          "(empty: the engine's)"},
+    {"q8_ks", "1", "Q8_0 matvecs of n_in <= 4096 below 65536 rows on the form without staging (0: never; 2, 4 or 8: "
+                   "that many rows a wave)"},
     {"ks", "1", "K-split matvec forms for n_in 4096 (Q4_K) and 12288 (Q6_K); 0: none; R_G: Q4_K shape"},
     {"ks6", "", "R_G_D: the Q6_K K-split form on that (rows, groups, groups ahead) shape"},
     {"ks3", "1", "the Q4_K K-split form for n_in 12288 (0: LDS-staged form; R_G: that shape)"},
@@ -255,6 +257,7 @@ struct MatvecAlt {
   uint64_t min_rows;
   uint32_t n_in_req = 0;              // nonzero: every segment's n_in must equal it
   uint64_t max_rows = ~uint64_t{0};   // and the launch at most this many rows
+  uint32_t n_in_over = ~0u;           // not ~0: instead every n_in above this and at most n_in_req
 };
 struct Retile {
   uint32_t n_out_word;     // index of n_out in the push words
@@ -409,7 +412,10 @@ Launch pack(const Command *const *run, uint32_t n) {
     for (const MatvecAlt &v : a.retile->alts) {
       if (rows < v.min_rows || rows > v.max_rows) continue;
       bool fits = true;
-      for (uint32_t i = 0; i < n && v.n_in_req; i++) fits &= run[i]->push[a.retile->n_in_word] == v.n_in_req;
+      for (uint32_t i = 0; i < n && v.n_in_req; i++) {
+        const uint32_t n_in = run[i]->push[a.retile->n_in_word];
+        fits &= v.n_in_over != ~0u ? n_in > v.n_in_over && n_in <= v.n_in_req : n_in == v.n_in_req;
+      }
       if (fits) {
         alt = &v;
         break;
@@ -1188,6 +1194,32 @@ void add_ks(skyla_hip_context *ctx, const char *name, const uint32_t *spec, Reti
       alts.push_back({fn, r.rpl * r.ng, 192, r.min_rows, 12288, r.max_rows});
     }
     t.n_in_word = 6;  // MatvecPush4.n_in
+    t.alts.insert(t.alts.end(), alts.begin(), alts.end());
+    return;
+  }
+  if (std::strncmp(name, "matvec_q8_0", 11) == 0 && spec[3] == 0 && tactic("q8_ks") != "0") {
+    // Q8_0 rows of at most 4096 values without staging (matvec_q8_0_ks_body): KW runs of 1024
+    // values, R rows a wave by the launch's rows, so that about 256 workgroups share a launch
+    // (the q8_ks tactic R forces one).  Six Qwen3-0.6B layers / a token, us: by rows 87.5 / 675,
+    // 2 everywhere 88.6 / 712, 4 88.5 / 688, 8 95.9 / 761, the LDS-staged form 110.7 / 798.  From
+    // 65536 rows (an output head) the lanes of q8_big read more bytes each than this form's
+    // activation loads cost.
+    const bool silu = std::strcmp(name, "matvec_q8_0_silu") == 0;
+    if (silu && spec[1] != 1) return;
+    const long forced = std::atol(tactic("q8_ks").c_str());
+    std::vector<MatvecAlt> alts;
+    for (uint32_t kw = 1; kw <= 4; kw++) {
+      const uint32_t rw = kw == 1 ? 4 : kw == 2 ? 2 : 1;
+      const struct { uint32_t r; uint64_t lo, hi; } rules[] = {
+          {2, 0, 256 * rw * 2}, {4, 256 * rw * 2 + 1, 256 * rw * 6}, {8, 256 * rw * 6 + 1, 65535}};
+      for (const auto &q : rules) {
+        const uint32_t r = forced == 2 || forced == 4 || forced == 8 ? (uint32_t)forced : q.r;
+        hipFunction_t fn = find_function(ctx, std::string(name) + "_ks__" + std::to_string(spec[1]) + "_" +
+                                                  std::to_string(kw) + "_" + std::to_string(r));
+        if (!fn) return;  // all or nothing
+        alts.push_back({fn, r * rw, 64 * kw * rw, q.lo, 1024 * kw, q.hi, 1024 * (kw - 1)});
+      }
+    }
     t.alts.insert(t.alts.end(), alts.begin(), alts.end());
     return;
   }
