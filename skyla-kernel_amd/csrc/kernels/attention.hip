@@ -533,6 +533,270 @@ SK_DEV void attention_body(const float *w, float *a, const uint32_t *ctl, f16 *k
   }
 }
 
+// attention of a batched step (attention_rows, the runtime's form of an attention grid of
+// several tokens): one wave per (kv head, split of CHUNK positions, 16 query rows), the rows
+// being N_REP heads of 16 / N_REP tokens.  It leaves the partials attention_body leaves.
+// One workgroup per token re-read the split's key and value rows (24 to 32 KB) for N_REP
+// rows and spent its time on staging, barriers and f32 FMAs; here both products run on the
+// matrix cores, the rows are read once per 16 queries, and nothing passes through LDS:
+//   S^T = K Q^T   A = key rows (row: position 16 t + c, c = lane % 16; dims 8 g + 32 k,
+//                 g = lane / 16), B = query rows, as loaded; a lane then holds query row c's
+//                 scores at positions 16 t + 4 g + r.
+//   O^T = V^T P^T B = that lane's own e values: a k-step's element j of group g is position
+//                 32 s + 16 (j / 4) + 4 g + j % 4.  A = value rows of those positions, lane c
+//                 holding dims 8 c + [0, 8) of each (whole rows a load); tile d takes dim
+//                 8 c + d as row c, so the transposition is 8 x 8 inside a lane.
+// Precision: query rows as f16 hi + lo of v 2^sh (put_q), e as hi + lo of e 2^14; f16 keys
+// and values and 8-bit keys are exact operands (8-bit keys' scales multiply each 32-dim
+// k-step's f32 sums), 8-bit values q s 2^vsh are 18 bits, exact as hi + lo: all products but
+// lo x lo (2^-22) in f32 sums.  Positions past a row's own have e = 0.  A split with a
+// value (or scale) that is not finite takes the values' non-finite elements in a product of
+// their own and zeroes, token by token, the rows past the token's position.
+template <int N_REP, int K8, int V8>
+SK_DEV void attention_rows_body(float *a, const uint32_t *ctl, const f16 *kv, const int8_t *kv8, const AttnPush &p,
+                                uint32_t n_grid) {
+  constexpr uint32_t TT = 16 / N_REP;
+  const uint32_t lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+  const uint32_t kvh = blockIdx.x, split = blockIdx.y, tok0 = blockIdx.z * TT, begin = split * CHUNK;
+  const uint32_t pos0 = ctl[1], n_tok = min(ctl[2], n_grid), kv_dim = p.n_kv * HD;
+  if (tok0 >= n_tok) return;
+  const uint32_t last = min(tok0 + TT, n_tok) - 1;  // the last live token of the group
+  if (begin >= pos0 + last + 1) return;
+  const uint32_t live = min(CHUNK, pos0 + last + 1 - begin);
+  // positions of this split that token t attends to
+  auto count = [&](uint32_t t) { return pos0 + t + 1 > begin ? min(CHUNK, pos0 + t + 1 - begin) : 0u; };
+  // this lane's query row (rows past the last live token repeat it and are not written)
+  const uint32_t tok = min(tok0 + c / N_REP, last), j = c % N_REP, cnt = count(tok);
+
+  uint4 kr[4][4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const uint32_t at = p.kc_off + (begin + min(16 * t + c, live - 1)) * kv_dim + kvh * HD + 8 * g;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if constexpr (K8) {
+        const uint2 r = *(const uint2 *)(kv8 + at + 32 * k);
+        kr[t][k] = make_uint4(r.x, r.y, 0u, 0u);
+      } else {
+        kr[t][k] = *(const uint4 *)(kv + at + 32 * k);
+      }
+    }
+  }
+  float4 qv[4][2];
+  const float *qrow = a + p.q_off + tok * p.q_stride + (kvh * N_REP + j) * HD + 8 * g;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    qv[k][0] = *(const float4 *)(qrow + 32 * k);
+    qv[k][1] = *(const float4 *)(qrow + 32 * k + 4);
+  }
+  f16x4 ks[4][4];  // 8-bit keys: the four block scales of positions 16 t + 4 g + r
+  if constexpr (K8)
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        ks[t][r] = *(const f16x4 *)(kv + p.ks_off + (begin + min(16 * t + 4 * g + r, live - 1)) * (kv_dim / 32) + kvh * 4);
+  uint4 vr[2][8];
+  float vs[2][8];
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint32_t vpos = begin + min(32 * s + 16 * (e >> 2) + 4 * g + (e & 3), live - 1);
+      const uint32_t at = p.vc_off + vpos * kv_dim + kvh * HD + 8 * c;
+      if constexpr (V8) {
+        const uint2 r = *(const uint2 *)(kv8 + at);
+        vr[s][e] = make_uint4(r.x, r.y, 0u, 0u);
+        vs[s][e] = (float)kv[p.vs_off + vpos * (kv_dim / 32) + kvh * 4 + (c >> 2)];
+      } else {
+        vr[s][e] = *(const uint4 *)(kv + at);
+        vs[s][e] = 1.0f;
+      }
+    }
+
+  // the query row's hi and lo parts
+  float q[4][8], big = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const float u[8] = {qv[k][0].x, qv[k][0].y, qv[k][0].z, qv[k][0].w, qv[k][1].x, qv[k][1].y, qv[k][1].z, qv[k][1].w};
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      q[k][e] = u[e] * p.scale;
+      big = fmaxf(big, fabsf(q[k][e]));
+    }
+  }
+  big = fmaxf(big, __shfl_xor(big, 16, 64));
+  big = fmaxf(big, __shfl_xor(big, 32, 64));
+  const int sh = big > 0.0f ? 11 - __builtin_amdgcn_frexp_expf(big) : 0;
+  f16x8 qh[4], ql[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float s = ldexpf(q[k][e], sh);
+      qh[k][e] = (f16)s;
+      ql[k][e] = (f16)(s - (float)qh[k][e]);
+    }
+
+  // two bytes picked by sel as an f16 pair: 1024 + (byte ^ 0x80), minus 1152
+  auto widen = [](uint32_t hi, uint32_t lo, uint32_t sel) {
+    const f16x2 off = {(f16)1152.0f, (f16)1152.0f};
+    return as_u32(as_f16x2((__builtin_amdgcn_perm(hi, lo, sel) ^ 0x00800080u) | 0x64006400u) - off);
+  };
+  float sc[4][4], m = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if constexpr (K8) {
+        const uint32_t x = kr[t][k].x, y = kr[t][k].y;
+        const uint4 w = make_uint4(widen(x, x, 0x0c010c00u), widen(x, x, 0x0c030c02u), widen(y, y, 0x0c010c00u),
+                                   widen(y, y, 0x0c030c02u));
+        f32x4 part = {0.0f, 0.0f, 0.0f, 0.0f};
+        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), ql[k], part, 0, 0, 0);
+        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), qh[k], part, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf((float)ks[t][r][k], part[r], acc[r]);
+      } else {
+        const f16x8 w = __builtin_bit_cast(f16x8, kr[t][k]);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, qh[k], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, ql[k], acc, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      sc[t][r] = 16 * t + 4 * g + r < cnt ? ldexpf(acc[r], -sh) : -INFINITY;
+      m = fmaxf(m, sc[t][r]);
+    }
+  }
+  m = fmaxf(m, __shfl_xor(m, 16, 64));
+  m = fmaxf(m, __shfl_xor(m, 32, 64));
+  float l = 0.0f;
+  f16x8 ph[2], pl[2], pn[2];  // e 2^14 as hi + lo; pn: 1 where e is not 0, for non-finite values
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float e = 16 * t + 4 * g + r < cnt ? expf(sc[t][r] - m) : 0.0f;
+      l += e;
+      const int s = t >> 1, i = 4 * (t & 1) + r;
+      const float x = e * 16384.0f;
+      ph[s][i] = (f16)x;
+      pl[s][i] = (f16)(x - (float)ph[s][i]);
+      pn[s][i] = e == 0.0f ? (f16)0.0f : (f16)(e / e);
+    }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+
+  // 8-bit values: the block's largest finite scale goes to [64, 128)
+  int vsh = 0;
+  bool odd = false;
+  if constexpr (V8) {
+    float top = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const bool fin = fabsf(vs[s][e]) < INFINITY;
+        odd |= !fin;
+        top = fmaxf(top, fin ? fabsf(vs[s][e]) : 0.0f);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    vsh = top > 0.0f ? 7 - __builtin_amdgcn_frexp_expf(top) : 0;
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) vs[s][e] = ldexpf(vs[s][e], vsh);
+  } else {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 top = {0, 0};
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const uint32_t u[4] = {vr[s][e].x, vr[s][e].y, vr[s][e].z, vr[s][e].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, u[i] & 0x7fff7fffu));
+      }
+    odd = top.x >= 0x7c00 || top.y >= 0x7c00;
+  }
+  auto word = [](const uint4 &u, int i) { return i == 0 ? u.x : i == 1 ? u.y : i == 2 ? u.z : u.w; };
+  // element d of value row e of k-step s, for 8-bit values with its scale
+  auto value = [&](int s, int e, int d) {
+    if constexpr (V8)
+      return (float)(int8_t)((word(vr[s][e], d >> 2) >> (8 * (d & 3))) & 255u) * vs[s][e];
+    else
+      return (float)__builtin_bit_cast(f16, (uint16_t)(word(vr[s][e], d >> 1) >> (16 * (d & 1))));
+  };
+  f32x4 o[8];
+#pragma unroll
+  for (int d = 0; d < 8; d++) o[d] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (__ballot(odd) == 0) {
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+      for (int d = 0; d < 8; d++) {
+        f16x8 vh, vl;
+        if constexpr (V8) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const float x = value(s, e, d);
+            vh[e] = (f16)x;
+            vl[e] = (f16)(x - (float)vh[e]);
+          }
+          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[s], o[d], 0, 0, 0);
+        } else {
+          const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
+          uint32_t u[4];
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            u[e] = __builtin_amdgcn_perm(word(vr[s][2 * e + 1], d >> 1), word(vr[s][2 * e], d >> 1), sel);
+          vh = __builtin_bit_cast(f16x8, make_uint4(u[0], u[1], u[2], u[3]));
+        }
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[s], o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[s], o[d], 0, 0, 0);
+      }
+  } else {
+    for (uint32_t tk = tok0; tk <= last; tk++) {
+      const uint32_t lim = count(tk);
+#pragma unroll
+      for (int d = 0; d < 8; d++) {
+        f32x4 x4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          f16x8 vh, vl, vn;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            const float x = 32 * s + 16 * (e >> 2) + 4 * g + (e & 3) < lim ? value(s, e, d) : 0.0f;
+            const bool fin = fabsf(x) < INFINITY;
+            vh[e] = (f16)(fin ? x : 0.0f);
+            vl[e] = (f16)(fin ? x - (float)vh[e] : 0.0f);
+            vn[e] = (f16)(fin ? 0.0f : x);
+          }
+          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[s], x4, 0, 0, 0);
+          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[s], x4, 0, 0, 0);
+          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[s], x4, 0, 0, 0);
+          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vn, pn[s], x4, 0, 0, 0);
+        }
+        if (tok == tk) o[d] = x4;
+      }
+    }
+  }
+  // row 4 g + r of tile d is dim 8 (4 g + r) + d, of block g
+  const int back = -14 - __shfl(vsh, (int)(4 * g), 64);
+  if (tok0 + c / N_REP > last || cnt == 0) return;
+  const uint32_t base = p.part_off + tok * p.part_stride + ((kvh * N_REP + j) * p.n_split + split) * PART;
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+#pragma unroll
+    for (int d = 0; d < 8; d += 2)
+      *(float2 *)(a + base + 2 + 8 * (4 * g + r) + d) = make_float2(ldexpf(o[d][r], back), ldexpf(o[d + 1][r], back));
+  if (g == 0) *(float2 *)(a + base) = make_float2(m, l);
+}
+
 }  // namespace
 
 // rmsnorm (rmsnorm.comp; ops.rs:1-16): y = x * r * w, r = 1 / sqrt(mean(x^2) + eps), per
@@ -609,6 +873,18 @@ QKV(1, 1)
 ATTN_REP(0, 0)
 ATTN_REP(0, 1)
 ATTN_REP(1, 1)
+
+#define ATTN_ROWS(R, K8, V8)                                                                     \
+  extern "C" __global__ __launch_bounds__(64) void attention_rows__##R##_64_##K8##_##V8##_128_128( \
+      float *a, const uint32_t *ctl, const f16 *kv, const int8_t *kv8, const f16 *kvs, AttnPush p,  \
+      uint32_t n_grid) {                                                                         \
+    (void)kvs;                                                                                   \
+    attention_rows_body<R, K8, V8>(a, ctl, kv, kv8, p, n_grid);                                  \
+  }
+#define ATTN_ROWS_REP(K8, V8) ATTN_ROWS(1, K8, V8) ATTN_ROWS(2, K8, V8) ATTN_ROWS(4, K8, V8) ATTN_ROWS(8, K8, V8)
+ATTN_ROWS_REP(0, 0)
+ATTN_ROWS_REP(0, 1)
+ATTN_ROWS_REP(1, 1)
 
 // attention_merge (attention_merge.comp): o = sum_s w_s acc_s / sum_s w_s l_s with
 // w_s = exp(m_s - max m) over the splits that hold positions.  Spec [head_dim, gated] =

@@ -98,6 +98,7 @@ const Tactic kTactics[] = {
     {"ring", "1", "dense matmuls on f16 rows take the ring tiles (0: never; WR_WK_NB_DX_S: that shape, split S ways)"},
     {"dl", "1", "matmul tiles with their operands loaded straight into LDS (0: register-staged)"},
     {"merge_t", "1", "batched attention merge as one wave per (head, token) (0: 1024-thread form)"},
+    {"attn_rows", "1", "attention of several tokens on the matrix cores, 16 query rows a wave (0: a workgroup per token)"},
     {"nograph", "0", "1: recordings replay as direct launches instead of one HIP graph (kernel traces)"},
 };
 
@@ -286,6 +287,7 @@ struct skyla_hip_pipeline {
   hipFunction_t tok_fn = nullptr;        // batched form: a tok_per_wg x tok_per_wg_y block of
   uint32_t tok_per_wg = 0;               // grid.x and grid.y per workgroup
   uint32_t tok_per_wg_y = 0;
+  uint32_t tok_per_wg_z = 0;             // attention: that many tokens (grid.z) per workgroup instead
   uint32_t tok_threads = 0;              // its workgroup size (0: the pipeline's)
   std::string name;                      // shader name
   hipFunction_t moe_fn = nullptr;        // MoE decode forms (fuse_moe), Q4_K experts: the gate/up pair,
@@ -308,7 +310,7 @@ struct Command {
                 hxms_fn = nullptr;
   std::shared_ptr<const RingFns> ring;
   hipFunction_t tok_fn = nullptr;
-  uint32_t tok_per_wg = 0, tok_per_wg_y = 0, tok_threads = 0;
+  uint32_t tok_per_wg = 0, tok_per_wg_y = 0, tok_per_wg_z = 0, tok_threads = 0;
   std::string name;                 // the pipeline's shader name
   hipFunction_t moe_fn = nullptr, moe_fn3 = nullptr, moe_fn4 = nullptr;
   uint32_t groups[3] = {0, 0, 0};
@@ -374,6 +376,15 @@ uint32_t split_of(const Command &a) {
   return S < 2 ? 1 : S;
 }
 
+// An attention grid of several tokens takes the matrix-core form (attention.hip,
+// attention_rows) where its wider accesses are aligned: query rows as float4, partials as
+// float2, the four block scales of an 8-bit row as one load (push words: AttnPush).  One
+// token keeps the form of four waves per split: a wave of 16 rows would hold N_REP.
+bool attention_rows_fit(const Command &a) {
+  const std::vector<uint32_t> &w = a.push;
+  return a.groups[2] > 1 && ((w[0] | w[7]) & 3u) == 0 && ((w[1] | w[8]) & 1u) == 0 && (w[9] & 3u) == 0;
+}
+
 // Packs consecutive dispatches of one segmented kernel into one launch.
 Launch pack(const Command *const *run, uint32_t n) {
   Launch l;
@@ -384,7 +395,14 @@ Launch pack(const Command *const *run, uint32_t n) {
   if (!a.segmented) {
     for (int i = 0; i < 3; i++) l.groups[i] = a.groups[i];
     l.args = a.push;
-    if (a.tok_fn && a.groups[1] > 1) {  // grid (x, y) = (experts, tokens): blocks of both
+    if (a.tok_fn && a.tok_per_wg_z) {
+      if (attention_rows_fit(a)) {
+        l.fn = a.tok_fn;
+        l.groups[2] = (a.groups[2] + a.tok_per_wg_z - 1) / a.tok_per_wg_z;
+        l.threads = a.tok_threads;
+        l.extra = {a.groups[2]};
+      }
+    } else if (a.tok_fn && a.groups[1] > 1) {  // grid (x, y) = (experts, tokens): blocks of both
       l.fn = a.tok_fn;
       l.groups[0] = (a.groups[0] + a.tok_per_wg - 1) / a.tok_per_wg;
       l.groups[1] = (a.groups[1] + a.tok_per_wg_y - 1) / a.tok_per_wg_y;
@@ -1082,6 +1100,7 @@ Command dispatch_command(const skyla_hip_pipeline *p, const std::vector<void *> 
   c.tok_fn = p->tok_fn;
   c.tok_per_wg = p->tok_per_wg;
   c.tok_per_wg_y = p->tok_per_wg_y;
+  c.tok_per_wg_z = p->tok_per_wg_z;
   c.tok_threads = p->tok_threads;
   c.name = p->name;
   c.moe_fn = p->moe_fn;
@@ -1608,6 +1627,13 @@ int skyla_hip_pipeline_new(skyla_hip_context *ctx, const char *name, uint32_t n_
       p->tok_per_wg_y = 1;
       p->tok_threads = 256;
     }
+  }
+  // the attention of a batched step: 16 query rows per wave, 16 / N_REP tokens (attention.hip,
+  // attention_rows); the attn_rows tactic 0 keeps one workgroup per token
+  if (std::strcmp(name, "attention") == 0 && n_spec == 6 && tactic_on("attn_rows")) {
+    p->tok_fn = find_function(ctx, "attention_rows" + sym.substr(std::strlen(name)));
+    p->tok_per_wg_z = 16 / spec[0];
+    p->tok_threads = 64;
   }
   // dense K-quant matmul (TYPE 1/2, MOE 0): its K-split variant, used for launches with few
   // tiles (split_of); the splitk tactic 0 keeps every launch on the engine's kernel
