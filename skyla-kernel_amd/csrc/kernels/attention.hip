@@ -982,16 +982,10 @@ extern "C" __global__ __launch_bounds__(1024) void attention_merge__128_0(float 
 // weights exp(m_s - M) are formed 64 at a time, one per lane, and broadcast by readlane (the
 // split index is wave-uniform).  The same quantity as attention_merge__128_0 in another
 // summation order; a prefill token has few splits, which the 1024-thread form leaves idle.
-extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float *a, const uint32_t *ctl,
-                                                                             MergePush p, uint32_t n_head,
-                                                                             uint32_t n_tok) {
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t h = blockIdx.x * 4 + wave, tok = blockIdx.y;
-  (void)n_tok;
-  if (tok >= ctl[2] || h >= n_head) return;
+SK_DEV float2 merge_head(const float *a, const uint32_t *ctl, const MergePush &p, uint32_t h, uint32_t tok,
+                         uint32_t lane) {
   const uint32_t used = min(min((ctl[1] + tok + p.chunk) / p.chunk, p.n_split), MAX_SPLITS);
   const uint32_t first = p.part_off + tok * p.part_stride + h * p.n_split * PART;
-  float *o = a + p.o_off + tok * p.o_stride + h * HD + 2 * lane;
   if (used <= 16) {
     // at most 16 splits (a prefill chunk within 1024 positions): every load in flight at
     // once, then the arithmetic below in the same order (the same bits)
@@ -1018,9 +1012,7 @@ extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float
         oy = __builtin_fmaf(wj, vy[j], oy);
       }
     total = wave_sum(total);
-    o[0] = ox / total;
-    o[1] = oy / total;
-    return;
+    return make_float2(ox / total, oy / total);
   }
   float big = -INFINITY;
   for (uint32_t s = lane; s < used; s += 64) big = fmaxf(big, a[first + s * PART]);
@@ -1039,8 +1031,78 @@ extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float
     }
   }
   total = wave_sum(total);
-  o[0] = ox / total;
-  o[1] = oy / total;
+  return make_float2(ox / total, oy / total);
+}
+extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float *a, const uint32_t *ctl,
+                                                                             MergePush p, uint32_t n_head,
+                                                                             uint32_t n_tok) {
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const uint32_t h = blockIdx.x * 4 + wave, tok = blockIdx.y;
+  (void)n_tok;
+  if (tok >= ctl[2] || h >= n_head) return;
+  const float2 v = merge_head(a, ctl, p, h, tok, lane);
+  float *o = a + p.o_off + tok * p.o_stride + h * HD + 2 * lane;
+  o[0] = v.x;
+  o[1] = v.y;
+}
+
+// attention_merge_t with the f16 row prepass of the matmul that reads its rows (o) in the same
+// launch: the f32 rows as attention_merge_t writes them, and each row's f16 values and
+// exponent at out as x_half_rows (matmul.hip) writes them: x 2^-e in the order 0, 2, 1, 3 of
+// every four, e = 0 unless the row's largest |x| reaches 2^15.  The row passes through LDS;
+// sixteen waves, a head each at a time (n_head <= MHEADS).  The separate prepass read back
+// what the launch before it wrote, its time mostly the launch's own.  Measured (MI355X, merge +
+// prepass -> one launch): 128 tokens of 32 heads at positions to 512 5.2 + 4.8 -> 8.1 us, 60
+// tokens of 16 heads in one split 4.5 + 4.3 -> 4.6 us.  Bound by a head's two dependent round
+// trips (with four waves a workgroup, eight heads each, the two launches were faster).
+// Grid: one workgroup per token.
+constexpr uint32_t MHEADS = 64;
+struct MergeHalfPush {
+  MergePush m;
+  uint32_t n_head, h_off;
+};
+extern "C" __global__ __launch_bounds__(1024) void attention_merge_half(float *a, uint32_t *out, const uint32_t *ctl,
+                                                                        MergeHalfPush q) {
+  __shared__ __attribute__((aligned(16))) float row[MHEADS * HD];
+  __shared__ float wm[16];
+  __shared__ uint32_t big[16];
+  const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63, tok = blockIdx.x;
+  const MergePush &p = q.m;
+  if (tok >= ctl[2]) return;
+  float m = 0.0f;
+  bool b = false;  // NaN counts as big, as in x_half_rows
+  for (uint32_t h = wave; h < q.n_head; h += 16) {
+    const float2 v = merge_head(a, ctl, p, h, tok, lane);
+    *(float2 *)(a + p.o_off + tok * p.o_stride + h * HD + 2 * lane) = v;
+    *(float2 *)&row[h * HD + 2 * lane] = v;
+    const float mh = fmaxf(fabsf(v.x), fabsf(v.y));
+    m = fmaxf(m, mh);
+    b |= !(mh < 32768.0f);
+  }
+  m = wave_max(m);
+  const uint64_t anyb = __ballot(b);
+  if (lane == 0) {
+    wm[wave] = m;
+    big[wave] = anyb != 0;
+  }
+  __syncthreads();
+  float tm = wm[0];
+  uint32_t any = big[0];
+#pragma unroll
+  for (int i = 1; i < 16; i++) {
+    tm = fmaxf(tm, wm[i]);
+    any |= big[i];
+  }
+  const int e = any && tm >= 32768.0f ? (int)((__builtin_bit_cast(uint32_t, tm) >> 23) & 255u) - 127 - 14 : 0;
+  const float sc = __builtin_ldexpf(1.0f, -e);
+  const uint32_t n = q.n_head * HD;
+  f16 *half = (f16 *)(out + q.h_off) + (size_t)tok * n;
+  for (uint32_t k = 4 * t; k < n; k += 4096) {
+    float4 v = *(const float4 *)&row[k];
+    if (e) v = make_float4(v.x * sc, v.y * sc, v.z * sc, v.w * sc);
+    *(uint2 *)(half + k) = make_uint2(as_u32(pack_f16x2(v.x, v.z)), as_u32(pack_f16x2(v.y, v.w)));
+  }
+  if (t == 0) out[tok] = (uint32_t)e;
 }
 
 // take_last (take_last.comp): the last token row of a chunk, for the output head.

@@ -1672,16 +1672,18 @@ struct XHalfPush {
 // e putting it below 2^15): the rows at out + h_off (f16 row t at t * n_in), pairs (0,2),
 // (1,3) of every four values as the tiles' LDS rows hold them; the exponent at out[t].
 constexpr int HALF_ROW_V = 48;  // values per thread: n_in <= 12288
-SK_DEV void store_half_row(const float4 (&v)[HALF_ROW_V / 4], uint32_t *out, uint32_t h_off, uint32_t n_in,
+template <int NT = 256>  // threads of the workgroup; 12288 values at 12288 / NT per thread
+SK_DEV void store_half_row(const float4 (&v)[HALF_ROW_V * 64 / NT], uint32_t *out, uint32_t h_off, uint32_t n_in,
                            uint32_t t) {
+  constexpr int V4 = HALF_ROW_V * 64 / NT, NW = NT / 64;
   const uint32_t tid = threadIdx.x;
   float m = 0.0f;
 #pragma unroll
-  for (int i = 0; i < HALF_ROW_V / 4; i++)
+  for (int i = 0; i < V4; i++)
     m = fmaxf(m, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
   // the row's largest |x| (NaN counts as big, as in the tile's guard)
-  __shared__ uint32_t big[4];
-  __shared__ float wm[4];
+  __shared__ uint32_t big[NW];
+  __shared__ float wm[NW];
   const bool b = !(m < 32768.0f);
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
@@ -1691,14 +1693,19 @@ SK_DEV void store_half_row(const float4 (&v)[HALF_ROW_V / 4], uint32_t *out, uin
     big[tid >> 6] = anyb != 0;
   }
   __syncthreads();
-  const float tm = fmaxf(fmaxf(wm[0], wm[1]), fmaxf(wm[2], wm[3]));
-  const bool any = big[0] | big[1] | big[2] | big[3];
+  float tm = wm[0];
+  uint32_t any = big[0];
+#pragma unroll
+  for (int i = 1; i < NW; i++) {
+    tm = fmaxf(tm, wm[i]);
+    any |= big[i];
+  }
   const int e = any && tm >= 32768.0f ? (int)((__builtin_bit_cast(uint32_t, tm) >> 23) & 255u) - 127 - 14 : 0;
   const float sc = __builtin_ldexpf(1.0f, -e);
   f16 *h = (f16 *)(out + h_off) + (size_t)t * n_in;
 #pragma unroll
-  for (int i = 0; i < HALF_ROW_V / 4; i++) {
-    const uint32_t k = 4 * (tid + 256 * i);
+  for (int i = 0; i < V4; i++) {
+    const uint32_t k = 4 * (tid + NT * i);
     if (k < n_in) {
       float4 a = v[i];
       if (e) a = make_float4(a.x * sc, a.y * sc, a.z * sc, a.w * sc);
@@ -1732,27 +1739,28 @@ extern "C" __global__ __launch_bounds__(256) void x_half_rows(const float *x, ui
 struct SiluHalfPush {
   uint32_t g_off, u_off, x_stride, n_in, h_off, rows_per_token;
 };
-extern "C" __global__ __launch_bounds__(256) void silu_half_rows(float *a, uint32_t *out, const uint32_t *ctl,
-                                                                 SiluHalfPush p) {
+template <int NT>
+SK_DEV void silu_half_body(float *a, uint32_t *out, const uint32_t *ctl, const SiluHalfPush &p) {
+  constexpr int V4 = HALF_ROW_V * 64 / NT;
   const uint32_t t = blockIdx.x, tid = threadIdx.x;
   if (t >= ctl[2] * p.rows_per_token) return;
   // every load in flight before the first is used: the passes the row needs (uniform), a
   // lane past the row's end reading its last four values (n_in is a multiple of 4)
-  const uint32_t n_pass = (p.n_in + 1023) / 1024;
+  const uint32_t n_pass = (p.n_in + 4 * NT - 1) / (4 * NT);
   float *gr = a + p.g_off + (size_t)t * p.x_stride;
   const float *ur = a + p.u_off + (size_t)t * p.x_stride;
-  float4 g[HALF_ROW_V / 4], u[HALF_ROW_V / 4];
+  float4 g[V4], u[V4];
 #pragma unroll
-  for (int i = 0; i < HALF_ROW_V / 4; i++)
+  for (int i = 0; i < V4; i++)
     if ((uint32_t)i < n_pass) {
-      const uint32_t k = min(4 * (tid + 256 * i), p.n_in - 4);
+      const uint32_t k = min(4 * (tid + NT * i), p.n_in - 4);
       g[i] = *(const float4 *)(gr + k);
       u[i] = *(const float4 *)(ur + k);
     }
-  float4 v[HALF_ROW_V / 4];
+  float4 v[V4];
 #pragma unroll
-  for (int i = 0; i < HALF_ROW_V / 4; i++) {
-    const uint32_t k = 4 * (tid + 256 * i);
+  for (int i = 0; i < V4; i++) {
+    const uint32_t k = 4 * (tid + NT * i);
     v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if ((uint32_t)i < n_pass && k < p.n_in) {
       {
@@ -1763,7 +1771,19 @@ extern "C" __global__ __launch_bounds__(256) void silu_half_rows(float *a, uint3
       *(float4 *)(gr + k) = v[i];
     }
   }
-  store_half_row(v, out, p.h_off, p.n_in, t);
+  store_half_row<NT>(v, out, p.h_off, p.n_in, t);
+}
+extern "C" __global__ __launch_bounds__(256) void silu_half_rows(float *a, uint32_t *out, const uint32_t *ctl,
+                                                                 SiluHalfPush p) {
+  silu_half_body<256>(a, out, ctl, p);
+}
+// A row a workgroup is 128 workgroups for a full chunk, half the CUs with one wave a SIMD: rows
+// of more than 4096 values (five passes and up of 256 threads) take sixteen waves.
+// 128 rows of 12288: 9.25 -> 7.76 us; up to 4096 values the four waves' passes are at most four
+// and in flight together (60 rows of 3072: 4.9 us, the launch's own time).
+extern "C" __global__ __launch_bounds__(1024) void silu_half_rows_wide(float *a, uint32_t *out, const uint32_t *ctl,
+                                                                       SiluHalfPush p) {
+  silu_half_body<1024>(a, out, ctl, p);
 }
 
 // rmsnorm (rmsnorm.comp; ops.rs:1-16) on the rows a dense matmul reads next, with that

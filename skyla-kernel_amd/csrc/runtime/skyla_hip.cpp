@@ -98,6 +98,8 @@ const Tactic kTactics[] = {
     {"ring", "1", "dense matmuls on f16 rows take the ring tiles (0: never; WR_WK_NB_DX_S: that shape, split S ways)"},
     {"dl", "1", "matmul tiles with their operands loaded straight into LDS (0: register-staged)"},
     {"merge_t", "1", "batched attention merge as one wave per (head, token) (0: 1024-thread form)"},
+    {"merge_join", "1", "the f16 row prepass of the matmul after a batched attention merge runs in the merge's launch "
+                        "(0: a launch of its own)"},
     {"attn_rows", "1", "attention of several tokens on the matrix cores, 16 query rows a wave (0: a workgroup per token)"},
     {"nograph", "0", "1: recordings replay as direct launches instead of one HIP graph (kernel traces)"},
 };
@@ -222,7 +224,9 @@ struct skyla_hip_context {
   uint32_t n_cu = 256;  // compute units of the device (hipDeviceProp_t.multiProcessorCount)
   hipFunction_t x_half_rows = nullptr;  // f16 row prepass of dense K-quant matmuls (matmul.hip)
   hipFunction_t silu_half_rows = nullptr;  // silu_mul with the expert down projection's prepass
+  hipFunction_t silu_half_wide = nullptr;  // the same in 1024 threads, for rows above 4096 values
   hipFunction_t silu_mul = nullptr;        // (moe.hip): the launch it replaces
+  hipFunction_t merge_t = nullptr, merge_half = nullptr;  // batched attention merge, and with the prepass
   hipFunction_t rmsnorm_half_rows = nullptr;  // rmsnorm with a dense matmul's prepass (matmul.hip)
   hipFunction_t rmsnorm = nullptr;            // (attention.hip): the launch it replaces
   std::shared_ptr<const RingFns> ring[3][2];  // the ring tiles by weight type and ACCUM
@@ -676,7 +680,7 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
   const bool x4 = xh != "8";       // 8: the eight-wave tile throughout
   const bool balance = xh != "4";  // 4: the plain grid
   const bool moe_xh = tactic_on("xhalf_moe");
-  const bool join = tactic_on("xhalf_join");
+  const bool join = tactic_on("xhalf_join"), merge_join = tactic_on("merge_join");
   uint32_t moe_used = 0;  // experts used per token: the x_div of the last expert gate/up matmul
   std::vector<Launch> out;
   std::vector<uint32_t> xkey;  // the rows the last prepass converted, until a barrier
@@ -801,8 +805,9 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
                                          a.push[4], a.push[8], a.push[6], a.groups[2]};
       if (key != xkey) {
         // The rows usually come from the launch just before: rmsnorm (q, k, v; gate and up)
-        // or silu_mul (down).  When it writes exactly these rows, one launch does both
-        // (rmsnorm_half_rows, silu_half_rows: the same f32 rows and the same f16 rows).
+        // or silu_mul (down) or the batched attention merge (o).  When it writes exactly these
+        // rows, one launch does both (rmsnorm_half_rows, silu_half_rows or, for rows above 4096
+        // values, silu_half_rows_wide, attention_merge_half: the same f32 and f16 rows).
         Launch f = x_half_prepass(ctx, a, h_off, rows);
         Launch *prev = out.empty() ? nullptr : &out.back();
         const bool plain = join && prev && !prev->mark && prev->split == 0 && prev->extra.empty() && prev->xh_buf < 0 &&
@@ -828,6 +833,24 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
           f.fn = ctx->silu_half_rows;
           f.bufs = {prev->bufs[0], nullptr, prev->bufs[1]};
           f.args = {prev->args[0], prev->args[1], a.push[8], a.push[6], (uint32_t)(h_off / 4), 1u};
+          if (ctx->silu_half_wide && a.push[6] > 4096) {
+            f.fn = ctx->silu_half_wide;
+            f.threads = 1024;
+          }
+          *prev = std::move(f);
+        } else if (merge_join && ctx->merge_half && prev && !prev->mark && prev->fn == ctx->merge_t && prev->args.size() == 6 &&
+                   prev->extra.size() == 2 && prev->bufs.size() == 2 && prev->bufs[0] == a.bufs[2] &&
+                   prev->bufs[1] == a.bufs[4] && prev->args[1] == a.push[4] && prev->args[5] == a.push[8] &&
+                   prev->extra[0] <= 64 && prev->extra[0] * 128 == a.push[6] && prev->extra[1] == rows &&
+                   ((prev->args[0] | prev->args[4]) & 1u) == 0) {
+          // MergePush + {n_head, h_off}; extra = {n_head, tokens} of the merge's grid
+          f.fn = ctx->merge_half;
+          f.threads = 1024;
+          f.bufs = {prev->bufs[0], nullptr, prev->bufs[1]};
+          f.args = prev->args;
+          f.args.push_back(prev->extra[0]);
+          f.args.push_back((uint32_t)(h_off / 4));
+          f.groups[0] = prev->extra[1];
           *prev = std::move(f);
         } else {
           out.push_back(std::move(f));
@@ -1410,6 +1433,9 @@ int skyla_hip_context_new(int device, skyla_hip_context **out) {
   }
   ctx->x_half_rows = find_function(ctx.get(), "x_half_rows");
   ctx->silu_half_rows = find_function(ctx.get(), "silu_half_rows");
+  ctx->silu_half_wide = find_function(ctx.get(), "silu_half_rows_wide");
+  ctx->merge_t = find_function(ctx.get(), "attention_merge_t__128_0");
+  ctx->merge_half = find_function(ctx.get(), "attention_merge_half");
   ctx->silu_mul = find_function(ctx.get(), "silu_mul");
   ctx->rmsnorm_half_rows = find_function(ctx.get(), "rmsnorm_half_rows");
   ctx->rmsnorm = find_function(ctx.get(), "rmsnorm");

@@ -1,0 +1,48 @@
+"""Prefill launches that carry the f16 row prepass of the matmul after them: the batched
+attention merge (attention_merge_half) and silu_mul in sixteen waves (silu_half_rows_wide, rows
+of more than 4096 values).  The same f32 and f16 rows as the separate launches, so the same
+logits bit for bit, over chunks with a ragged end and contexts of several splits."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from helpers import tactics
+from skyla_hip import engine as E
+from skyla_hip import synth
+
+pytestmark = pytest.mark.gpu
+
+CFG = "test-prefill-joins"
+
+
+def _logits(ctx, c, tensors, prompt, **tactic):
+    with tactics(**tactic):
+        eng = E.Engine(ctx, tensors, c, 40 * E.ATTENTION_CHUNK, E.KvPrecision.F16_KEYS_Q8_VALUES)
+        try:
+            rows = [eng.prefill(prompt).copy(), eng.step(int(prompt[0])).copy()]
+            return np.stack(rows).view(np.uint32), eng.recording(True, E.BATCH).launches()
+        finally:
+            eng.free()
+
+
+# one chunk of one row; a ragged second chunk; more than 16 splits (the merge's other loop)
+@pytest.mark.parametrize("n_prompt", [2, E.BATCH + 22, 17 * E.ATTENTION_CHUNK + 5])
+def test_merge_with_prepass_same_logits(ctx, n_prompt):
+    c = synth.qwen3_config("tiny")
+    tensors = synth.qwen3(CFG, c, "q4_k_m", "random")
+    prompt = synth.prompt(f"{CFG}-{n_prompt}", n_prompt, c.n_vocab)
+    got, n1 = _logits(ctx, c, tensors, prompt)
+    want, n0 = _logits(ctx, c, tensors, prompt, merge_join="0")
+    assert n0 - n1 == c.n_layer and np.array_equal(got, want)
+
+
+# either side of the line at 4096 values, and the longest rows (12288: three full passes)
+@pytest.mark.parametrize("n_ff", [4096, 4352, 12288])
+def test_wide_silu_with_prepass_same_logits(ctx, n_ff):
+    c = dataclasses.replace(synth.qwen3_config("tiny"), n_ff=n_ff)
+    tensors = synth.qwen3(f"{CFG}-{n_ff}", c, "q4_k_m", "random")
+    prompt = synth.prompt(f"{CFG}-ff", 45, c.n_vocab)
+    got, n1 = _logits(ctx, c, tensors, prompt)
+    want, n0 = _logits(ctx, c, tensors, prompt, xhalf_join="0")
+    assert n0 > n1 and np.array_equal(got, want)
