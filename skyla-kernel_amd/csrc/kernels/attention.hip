@@ -538,7 +538,8 @@ SK_DEV void attention_body(const float *w, float *a, const uint32_t *ctl, f16 *k
 // being N_REP heads of 16 / N_REP tokens.  It leaves the partials attention_body leaves.
 // One workgroup per token re-read the split's key and value rows (24 to 32 KB) for N_REP
 // rows and spent its time on staging, barriers and f32 FMAs; here both products run on the
-// matrix cores, the rows are read once per 16 queries, and nothing passes through LDS:
+// matrix cores, the rows are read once per 16 queries, and nothing passes through LDS (but in
+// the rare splits taken in f32, below):
 //   S^T = K Q^T   A = key rows (row: position 16 t + c, c = lane % 16; dims 8 g + 32 k,
 //                 g = lane / 16), B = query rows, as loaded; a lane then holds query row c's
 //                 scores at positions 16 t + 4 g + r.
@@ -546,14 +547,21 @@ SK_DEV void attention_body(const float *w, float *a, const uint32_t *ctl, f16 *k
 //                 32 s + 16 (j / 4) + 4 g + j % 4.  A = value rows of those positions, lane c
 //                 holding dims 8 c + [0, 8) of each (whole rows a load); tile d takes dim
 //                 8 c + d as row c, so the transposition is 8 x 8 inside a lane.
-// Precision: query rows as f16 hi + lo of v 2^sh (put_q), e as hi + lo of e 2^14; f16 keys
-// and values and 8-bit keys are exact operands (8-bit keys' scales multiply each 32-dim
-// k-step's f32 sums), 8-bit values q s 2^vsh are 18 bits, exact as hi + lo: all products but
-// lo x lo (2^-22) in f32 sums.  Positions past a row's own have e = 0.  A split with a
-// value (or scale) that is not finite takes the values' non-finite elements in a product of
-// their own and zeroes, token by token, the rows past the token's position.
+// Precision: what attention_body holds in f32 keeps its 24 bits, as three f16 parts of 11: e 2^15
+// (exact from e = 2^-16 of the split's largest, below that to 2^-40) and, over 8-bit keys, the
+// query rows v 2^sh (to 2^-39 of the row's largest); over f16 keys the rows are hi + lo, as put_q
+// has them.  f16 keys and values and 8-bit keys are exact operands (8-bit keys' scales multiply
+// each 32-dim k-step's f32 sums); 8-bit values q s are 18 bits, exact as hi + lo of q s 2^vsh while
+// the scales of a block's positions lie within 2^20 of its largest.  Only the product of the last
+// parts (2^-33) is left out; sums are f32.  Positions past a row's own have e = 0.  A split with
+// scales further apart, or with a value or scale that is not finite, takes its values in f32
+// (attention_body's arithmetic), each row over its own positions alone.
+// Error against 64 bits over attention_body's on the same inputs, N(0, 1) rows at positions to
+// 1517 in every precision, queries of N(0, 1), 8 times that, or spread over 2^12: 0.83 to 1.005
+// (with two parts of e and of the query rows and no product of the low parts 0.93 to 1.12, and
+// 0.6 us less a launch at most).
 // Measured (MI355X, a launch): 128 tokens of Qwen3-8B at positions to 512, f16 keys and 8-bit
-// values, 25.9 -> 12.3 us; 60 tokens of Qwen3-0.6B in f16 5.8 -> 5.3 us.  All a wave's loads
+// values, 25.9 -> 12.3 us; 60 tokens of Qwen3-0.6B in f16 5.8 -> 5.7 us.  All a wave's loads
 // are in flight at once, which two waves a SIMD (256 registers) hold; with one (288 to 320
 // registers) and the value loads behind the scores the former ran 16.0 us.  Bound by the
 // round trip and, with several waves a SIMD, by the values' conversion and the partials' writes.
@@ -635,15 +643,17 @@ SK_DEV void attention_rows_body(float *a, const uint32_t *ctl, const f16 *kv, co
   }
   big = fmaxf(big, __shfl_xor(big, 16, 64));
   big = fmaxf(big, __shfl_xor(big, 32, 64));
-  const int sh = big > 0.0f ? 11 - __builtin_amdgcn_frexp_expf(big) : 0;
-  f16x8 qh[4], ql[4];
+  const int sh = big > 0.0f ? (K8 ? 15 : 11) - __builtin_amdgcn_frexp_expf(big) : 0;
+  f16x8 qh[4], ql[4], qt[4];  // qt: the third part (8-bit keys)
 #pragma unroll
   for (int k = 0; k < 4; k++)
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       const float s = ldexpf(q[k][e], sh);
       qh[k][e] = (f16)s;
-      ql[k][e] = (f16)(s - (float)qh[k][e]);
+      const float r = s - (float)qh[k][e];
+      ql[k][e] = (f16)r;
+      if constexpr (K8) qt[k][e] = (f16)(r - (float)ql[k][e]);
     }
 
   // two bytes picked by sel as an f16 pair: 1024 + (byte ^ 0x80), minus 1152
@@ -662,6 +672,7 @@ SK_DEV void attention_rows_body(float *a, const uint32_t *ctl, const f16 *kv, co
         const uint4 w = make_uint4(widen(x, x, 0x0c010c00u), widen(x, x, 0x0c030c02u), widen(y, y, 0x0c010c00u),
                                    widen(y, y, 0x0c030c02u));
         f32x4 part = {0.0f, 0.0f, 0.0f, 0.0f};
+        part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), qt[k], part, 0, 0, 0);
         part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), ql[k], part, 0, 0, 0);
         part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), qh[k], part, 0, 0, 0);
 #pragma unroll
@@ -683,23 +694,19 @@ SK_DEV void attention_rows_body(float *a, const uint32_t *ctl, const f16 *kv, co
   // a masked score is -inf and its e is 0 without a branch (a row without positions is not written)
   const float mu = cnt ? m : 0.0f;
   float l = 0.0f;
-  f16x8 ph[2], pl[2], pn[2];  // e 2^14 as hi + lo; pn: 1 where e is not 0, for non-finite values
 #pragma unroll
   for (int t = 0; t < 4; t++)
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const float e = expf(sc[t][r] - mu);
-      l += e;
-      const int s = t >> 1, i = 4 * (t & 1) + r;
-      const float x = e * 16384.0f;
-      ph[s][i] = (f16)x;
-      pl[s][i] = (f16)(x - (float)ph[s][i]);
-      pn[s][i] = (f16)(e > 0.0f ? 1.0f : e);
+      sc[t][r] = expf(sc[t][r] - mu);
+      l += sc[t][r];
     }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
+  const bool writes = tok0 + c / N_REP <= last && cnt != 0;
+  const uint32_t base = p.part_off + tok * p.part_stride + ((kvh * N_REP + j) * p.n_split + split) * PART;
 
-  // 8-bit values: the block's largest finite scale goes to [64, 128)
+  // 8-bit values: the block's largest finite scale goes to [64, 128).  odd: the split takes f32
   int vsh = 0;
   bool odd = false;
   if constexpr (V8) {
@@ -719,7 +726,11 @@ SK_DEV void attention_rows_body(float *a, const uint32_t *ctl, const f16 *kv, co
 #pragma unroll
     for (int s = 0; s < 2; s++)
 #pragma unroll
-      for (int e = 0; e < 8; e++) vs[s][e] = (f16)ldexpf((float)vs[s][e], vsh);
+      for (int e = 0; e < 8; e++) {
+        const float x = ldexpf((float)vs[s][e], vsh);
+        vs[s][e] = (f16)x;
+        odd |= (float)vs[s][e] != x;  // too far below the block's largest
+      }
   } else {
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     u16x2 top = {0, 0};
@@ -734,76 +745,106 @@ SK_DEV void attention_rows_body(float *a, const uint32_t *ctl, const f16 *kv, co
       }
     odd = top.x >= 0x7c00 || top.y >= 0x7c00;
   }
+  if (__ballot(odd)) {
+    // row i's e at [position][i]; lane: dims 2 lane, 2 lane + 1 of every row
+    __shared__ float es[CHUNK][16];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) es[16 * t + 4 * g + r][c] = sc[t][r];
+    __syncthreads();
+    float ox[16], oy[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) ox[i] = oy[i] = 0.0f;
+    for (uint32_t n = 0; n < live; n++) {
+      const uint32_t pos = begin + n, at = p.vc_off + pos * kv_dim + kvh * HD + 2 * lane;
+      float vx, vy;
+      if constexpr (V8) {
+        const float s = (float)kv[p.vs_off + pos * (kv_dim / 32) + kvh * 4 + (lane >> 4)];
+        vx = (float)kv8[at] * s;
+        vy = (float)kv8[at + 1] * s;
+      } else {
+        vx = (float)kv[at];
+        vy = (float)kv[at + 1];
+      }
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        if (n < count(tok0 + i / N_REP)) {
+          ox[i] = __builtin_fmaf(es[n][i], vx, ox[i]);
+          oy[i] = __builtin_fmaf(es[n][i], vy, oy[i]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const uint32_t tk = tok0 + i / N_REP;
+      if (tk <= last && count(tk) != 0)
+        *(float2 *)(a + p.part_off + tk * p.part_stride + ((kvh * N_REP + i % N_REP) * p.n_split + split) * PART + 2 +
+                    2 * lane) = make_float2(ox[i], oy[i]);
+    }
+    if (g == 0 && writes) *(float2 *)(a + base) = make_float2(m, l);
+    return;
+  }
+  f16x8 ph[2], pm[2], pl[2];  // e 2^15 in three parts
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int s = t >> 1, i = 4 * (t & 1) + r;
+      const float x = sc[t][r] * 32768.0f;
+      ph[s][i] = (f16)x;
+      const float y = x - (float)ph[s][i];
+      pm[s][i] = (f16)y;
+      pl[s][i] = (f16)(y - (float)pm[s][i]);
+    }
   auto word = [](const uint4 &u, int i) { return i == 0 ? u.x : i == 1 ? u.y : i == 2 ? u.z : u.w; };
-  // element d of value row e of k-step s, for 8-bit values with its scale
-  auto value = [&](int s, int e, int d) {
-    if constexpr (V8)
-      return (float)(int8_t)((word(vr[s][e], d >> 2) >> (8 * (d & 3))) & 255u) * (float)vs[s][e];
-    else
-      return (float)__builtin_bit_cast(f16, (uint16_t)(word(vr[s][e], d >> 1) >> (16 * (d & 1))));
-  };
   f32x4 o[8];
 #pragma unroll
   for (int d = 0; d < 8; d++) o[d] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (__ballot(odd) == 0) {
 #pragma unroll
-    for (int s = 0; s < 2; s++)
+  for (int d = 0; d < 8; d++) {
+    f16x8 vh[2], vl[2];
 #pragma unroll
-      for (int d = 0; d < 8; d++) {
-        f16x8 vh, vl;
-        if constexpr (V8) {
+    for (int s = 0; s < 2; s++) {
+      if constexpr (V8) {
 #pragma unroll
-          for (int e = 0; e < 8; e += 2) {
-            // q s rounded once, and what that left (exact): two packed operations a pair
-            const uint32_t at = d & 3, sel = 0x0c040c00u + at * 0x00010001u;
-            const f16x2 v = as_f16x2(widen(word(vr[s][e + 1], d >> 2), word(vr[s][e], d >> 2), sel));
-            const f16x2 sv = {(f16)vs[s][e], (f16)vs[s][e + 1]};
-            const f16x2 hi = v * sv, lo = __builtin_elementwise_fma(v, sv, -hi);
-            vh[e] = hi.x, vh[e + 1] = hi.y;
-            vl[e] = lo.x, vl[e + 1] = lo.y;
-          }
-          o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[s], o[d], 0, 0, 0);
-        } else {
-          const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
-          uint32_t u[4];
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            u[e] = __builtin_amdgcn_perm(word(vr[s][2 * e + 1], d >> 1), word(vr[s][2 * e], d >> 1), sel);
-          vh = __builtin_bit_cast(f16x8, make_uint4(u[0], u[1], u[2], u[3]));
+        for (int e = 0; e < 8; e += 2) {
+          // q s rounded once, and what that left (exact): two packed operations a pair
+          const uint32_t at = d & 3, sel = 0x0c040c00u + at * 0x00010001u;
+          const f16x2 v = as_f16x2(widen(word(vr[s][e + 1], d >> 2), word(vr[s][e], d >> 2), sel));
+          const f16x2 sv = {vs[s][e], vs[s][e + 1]};
+          const f16x2 hi = v * sv, lo = __builtin_elementwise_fma(v, sv, -hi);
+          vh[s][e] = hi.x, vh[s][e + 1] = hi.y;
+          vl[s][e] = lo.x, vl[s][e + 1] = lo.y;
         }
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[s], o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[s], o[d], 0, 0, 0);
-      }
-  } else {
-    for (uint32_t tk = tok0; tk <= last; tk++) {
-      const uint32_t lim = count(tk);
+      } else {
+        const uint32_t sel = d & 1 ? 0x07060302u : 0x05040100u;
+        uint32_t u[4];
 #pragma unroll
-      for (int d = 0; d < 8; d++) {
-        f32x4 x4 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-          f16x8 vh, vl, vn;
-#pragma unroll
-          for (int e = 0; e < 8; e++) {
-            const float x = 32 * s + 16 * (e >> 2) + 4 * g + (e & 3) < lim ? value(s, e, d) : 0.0f;
-            const bool fin = fabsf(x) < INFINITY;
-            vh[e] = (f16)(fin ? x : 0.0f);
-            vl[e] = (f16)(fin ? x - (float)vh[e] : 0.0f);
-            vn[e] = (f16)(fin ? 0.0f : x);
-          }
-          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[s], x4, 0, 0, 0);
-          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[s], x4, 0, 0, 0);
-          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[s], x4, 0, 0, 0);
-          x4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(vn, pn[s], x4, 0, 0, 0);
-        }
-        if (tok == tk) o[d] = x4;
+        for (int e = 0; e < 4; e++)
+          u[e] = __builtin_amdgcn_perm(word(vr[s][2 * e + 1], d >> 1), word(vr[s][2 * e], d >> 1), sel);
+        vh[s] = __builtin_bit_cast(f16x8, make_uint4(u[0], u[1], u[2], u[3]));
       }
     }
+    // the smallest products first: the sum rounds at its full size twice
+    auto add = [&](const f16x8 &v, const f16x8 &e) {
+      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, e, o[d], 0, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < 2; s++) add(vh[s], pl[s]);
+    if constexpr (V8)
+#pragma unroll
+      for (int s = 0; s < 2; s++) add(vl[s], pm[s]);
+#pragma unroll
+    for (int s = 0; s < 2; s++) add(vh[s], pm[s]);
+    if constexpr (V8)
+#pragma unroll
+      for (int s = 0; s < 2; s++) add(vl[s], ph[s]);
+#pragma unroll
+    for (int s = 0; s < 2; s++) add(vh[s], ph[s]);
   }
   // row 4 g + r of tile d is dim 8 (4 g + r) + d, of block g
-  const int back = -14 - __shfl(vsh, (int)(4 * g), 64);
-  if (tok0 + c / N_REP > last || cnt == 0) return;
-  const uint32_t base = p.part_off + tok * p.part_stride + ((kvh * N_REP + j) * p.n_split + split) * PART;
+  const int back = -15 - __shfl(vsh, (int)(4 * g), 64);
+  if (!writes) return;
 #pragma unroll
   for (int r = 0; r < 4; r++)
 #pragma unroll
