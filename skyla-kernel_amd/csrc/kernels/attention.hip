@@ -20,7 +20,7 @@
 // at vc_off; an 8-bit row keeps one f16 scale per 32 values at
 // scales + pos * kv_dim / 32 + head * 4 + block.  An entry is quantised as
 // s = max|y| over its block / 127, q = round(y / s) (qkv_prep.comp:44-65; ties to even).
-#include "common.h"
+#include "matmul_common.h"
 
 namespace {
 
@@ -1089,9 +1089,9 @@ extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float
 
 // attention_merge_t with the f16 row prepass of the matmul that reads its rows (o) in the same
 // launch: the f32 rows as attention_merge_t writes them, and each row's f16 values and
-// exponent at out as x_half_rows (matmul.hip) writes them: x 2^-e in the order 0, 2, 1, 3 of
-// every four, e = 0 unless the row's largest |x| reaches 2^15.  The row passes through LDS;
-// sixteen waves, a head each at a time (n_head <= MHEADS).  The separate prepass read back
+// exponent (or the runs' exponents) at out as x_half_rows (matmul.hip) writes them: x 2^-e in the
+// order 0, 2, 1, 3 of every four, e = 0 unless the row's largest |x| reaches 2^15.  The row
+// passes through LDS; sixteen waves, a head each at a time (n_head <= MHEADS).  The separate prepass read back
 // what the launch before it wrote, its time mostly the launch's own.  Measured (MI355X, merge +
 // prepass -> one launch): 128 tokens of 32 heads at positions to 512 5.2 + 4.8 -> 8.1 us, 60
 // tokens of 16 heads in one split 4.5 + 4.3 -> 4.6 us.  Bound by a head's two dependent round
@@ -1100,7 +1100,7 @@ extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float
 constexpr uint32_t MHEADS = 64;
 struct MergeHalfPush {
   MergePush m;
-  uint32_t n_head, h_off;
+  uint32_t n_head, h_off, e_off;
 };
 extern "C" __global__ __launch_bounds__(1024) void attention_merge_half(float *a, uint32_t *out, const uint32_t *ctl,
                                                                         MergeHalfPush q) {
@@ -1134,12 +1134,17 @@ extern "C" __global__ __launch_bounds__(1024) void attention_merge_half(float *a
     tm = fmaxf(tm, wm[i]);
     any |= big[i];
   }
-  const int e = any && tm >= 32768.0f ? (int)((__builtin_bit_cast(uint32_t, tm) >> 23) & 255u) - 127 - 14 : 0;
-  const float sc = __builtin_ldexpf(1.0f, -e);
+  const int e = any ? range_exp(tm) : 0;
+  float sc = __builtin_ldexpf(1.0f, -e);
   const uint32_t n = q.n_head * HD;
   f16 *half = (f16 *)(out + q.h_off) + (size_t)tok * n;
   for (uint32_t k = 4 * t; k < n; k += 4096) {
     float4 v = *(const float4 *)&row[k];
+    if (e && q.e_off) {  // an exponent per run of 128 values (n is a multiple of 128)
+      const int er = run_exp(v);
+      sc = __builtin_ldexpf(1.0f, -er);
+      if ((t & 31) == 0) out[q.e_off + tok * (n / E_RUN) + k / E_RUN] = (uint32_t)er;
+    }
     if (e) v = make_float4(v.x * sc, v.y * sc, v.z * sc, v.w * sc);
     *(uint2 *)(half + k) = make_uint2(as_u32(pack_f16x2(v.x, v.z)), as_u32(pack_f16x2(v.y, v.w)));
   }

@@ -1662,19 +1662,23 @@ MMHS(2, 1)
 // multiplies its sums back by 2^e_t.  With e_t = 0 the f16 values, and so the GEMM's bits,
 // are those of the tile's own conversion (round to nearest even).  Grid: one workgroup per
 // row of the launch's token tiles; out = [e: one int32 per row][rows: f16 from u32 h_off,
-// n_in per row, 16-byte aligned].
+// n_in per row, 16-byte aligned].  With e_off (rows for the Q8_0 ring tile) each run of 128
+// values has its own exponent, as the Q8_0 tile's own staging has: e[t] is nonzero where a run's
+// is, and then row t's are at u32 e_off + t * ceil(n_in / 128).
 struct XHalfPush {
   uint32_t x_off, x_stride, n_in, h_off;
   uint32_t rows_per_token;  // input rows per token of ctl[2]: 1, or the slots of an expert down
+  uint32_t e_off;           // 0, or where the runs' exponents go
 };
 // One row of f16 for the tiles from its values v (n_in <= 12288 at 4 per thread and 256
 // threads), with e = 0 unless the row's largest |x| reaches 2^15 (then the row is x * 2^-e,
 // e putting it below 2^15): the rows at out + h_off (f16 row t at t * n_in), pairs (0,2),
-// (1,3) of every four values as the tiles' LDS rows hold them; the exponent at out[t].
+// (1,3) of every four values as the tiles' LDS rows hold them; the exponent at out[t].  e_off: an
+// exponent per run of 128 values (x_half_rows).
 constexpr int HALF_ROW_V = 48;  // values per thread: n_in <= 12288
 template <int NT = 256>  // threads of the workgroup; 12288 values at 12288 / NT per thread
 SK_DEV void store_half_row(const float4 (&v)[HALF_ROW_V * 64 / NT], uint32_t *out, uint32_t h_off, uint32_t n_in,
-                           uint32_t t) {
+                           uint32_t t, uint32_t e_off) {
   constexpr int V4 = HALF_ROW_V * 64 / NT, NW = NT / 64;
   const uint32_t tid = threadIdx.x;
   float m = 0.0f;
@@ -1700,17 +1704,26 @@ SK_DEV void store_half_row(const float4 (&v)[HALF_ROW_V * 64 / NT], uint32_t *ou
     tm = fmaxf(tm, wm[i]);
     any |= big[i];
   }
-  const int e = any && tm >= 32768.0f ? (int)((__builtin_bit_cast(uint32_t, tm) >> 23) & 255u) - 127 - 14 : 0;
-  const float sc = __builtin_ldexpf(1.0f, -e);
+  const int e = any ? range_exp(tm) : 0;
   f16 *h = (f16 *)(out + h_off) + (size_t)t * n_in;
-#pragma unroll
-  for (int i = 0; i < V4; i++) {
+  auto put = [&](int i, float sc) {
     const uint32_t k = 4 * (tid + NT * i);
-    if (k < n_in) {
-      float4 a = v[i];
-      if (e) a = make_float4(a.x * sc, a.y * sc, a.z * sc, a.w * sc);
-      *(uint2 *)(h + k) = make_uint2(as_u32(pack_f16x2(a.x, a.z)), as_u32(pack_f16x2(a.y, a.w)));
+    if (k < n_in)
+      *(uint2 *)(h + k) = make_uint2(as_u32(pack_f16x2(v[i].x * sc, v[i].z * sc)),
+                                     as_u32(pack_f16x2(v[i].y * sc, v[i].w * sc)));
+  };
+  if (__builtin_expect(e && e_off, 0)) {
+#pragma unroll
+    for (int i = 0; i < V4; i++) {
+      const uint32_t k = 4 * (tid + NT * i);
+      const int er = run_exp(v[i]);
+      if ((tid & 31) == 0 && k < n_in) out[e_off + t * ((n_in + E_RUN - 1) / E_RUN) + k / E_RUN] = (uint32_t)er;
+      put(i, __builtin_ldexpf(1.0f, -er));
     }
+  } else {
+    const float sc = __builtin_ldexpf(1.0f, -e);
+#pragma unroll
+    for (int i = 0; i < V4; i++) put(i, sc);
   }
   if (tid == 0) out[t] = (uint32_t)e;
 }
@@ -1727,7 +1740,7 @@ extern "C" __global__ __launch_bounds__(256) void x_half_rows(const float *x, ui
     v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (k < p.n_in) v[i] = *(const float4 *)(xr + k);
   }
-  store_half_row(v, out, p.h_off, p.n_in, t);
+  store_half_row(v, out, p.h_off, p.n_in, t, p.e_off);
 }
 
 // silu_mul (silu_mul.comp:15-23) on the rows an expert down projection reads, with that
@@ -1737,7 +1750,7 @@ extern "C" __global__ __launch_bounds__(256) void x_half_rows(const float *x, ui
 // past n_in of a row and the rows past the slots are not computed: no later launch reads
 // them.
 struct SiluHalfPush {
-  uint32_t g_off, u_off, x_stride, n_in, h_off, rows_per_token;
+  uint32_t g_off, u_off, x_stride, n_in, h_off, rows_per_token, e_off;
 };
 template <int NT>
 SK_DEV void silu_half_body(float *a, uint32_t *out, const uint32_t *ctl, const SiluHalfPush &p) {
@@ -1771,7 +1784,7 @@ SK_DEV void silu_half_body(float *a, uint32_t *out, const uint32_t *ctl, const S
       *(float4 *)(gr + k) = v[i];
     }
   }
-  store_half_row<NT>(v, out, p.h_off, p.n_in, t);
+  store_half_row<NT>(v, out, p.h_off, p.n_in, t, p.e_off);
 }
 extern "C" __global__ __launch_bounds__(256) void silu_half_rows(float *a, uint32_t *out, const uint32_t *ctl,
                                                                  SiluHalfPush p) {
@@ -1795,7 +1808,7 @@ extern "C" __global__ __launch_bounds__(1024) void silu_half_rows_wide(float *a,
 struct NormHalfPush {
   uint32_t x_off, w_off, y_off, n;
   float eps;
-  uint32_t stride, h_off;
+  uint32_t stride, h_off, e_off;
 };
 extern "C" __global__ __launch_bounds__(256) void rmsnorm_half_rows(const float *w, float *a, uint32_t *out,
                                                                     const uint32_t *ctl, NormHalfPush p) {
@@ -1812,7 +1825,7 @@ extern "C" __global__ __launch_bounds__(256) void rmsnorm_half_rows(const float 
     v[k] = y4[k];
     if (t + 256 * k < (p.n >> 2)) yr[t + 256 * k] = y4[k];
   }
-  store_half_row(v, out, p.h_off, p.n, tok);
+  store_half_row(v, out, p.h_off, p.n, tok, p.e_off);
 }
 
 // Workspace of skyla_hip_dispatch_noalloc, the entry point that allocates nothing: the K

@@ -65,6 +65,21 @@ SK_DEV void step_scale(const WStage<TYPE> &s, int t, uint32_t hh, f16x2 &scale, 
   }
 }
 
+// f16 range guard: rows reaching |x| = tm are held as x 2^-e, e putting tm below 2^15.
+SK_DEV int range_exp(float tm) {
+  return tm >= 32768.0f ? (int)((__builtin_bit_cast(uint32_t, tm) >> 23) & 255u) - 127 - 14 : 0;
+}
+// The same for each E_RUN values of a row (Q8_0 rows, whose tile rescales its sums between runs:
+// one exponent for a row would flush what lies 2^29 below its largest).  v: four values per lane,
+// 32 lanes a run.
+constexpr uint32_t E_RUN = 128;
+SK_DEV int run_exp(const float4 &v) {
+  float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+#pragma unroll
+  for (int d = 16; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+  return range_exp(m);
+}
+
 // 16 B unit slot swizzle of a direct-to-LDS row (128 B rows, 8 units): distinct banks for 16
 // consecutive rows in a 256 B bank line and for 8 in a 128 B one
 SK_DEV uint32_t dl_swz(uint32_t r) { return (r & 7u) ^ ((r >> 3) & 1u); }

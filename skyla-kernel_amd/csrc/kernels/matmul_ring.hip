@@ -15,6 +15,11 @@
 //           scales 16 B, and the 16 B around the row's d, per super-block
 //     Q8_0  64 B of quants per row and chunk at 64 r (units ^ (r >> 2) & 3); the two 16 B pieces
 //           that hold the row's eight d (2 B-aligned), per 256 k
+// Exponents (|x| reaching 2^15): rows of K-quant matrices have one each, by which the sums are
+// scaled at the end.  Rows of Q8_0 matrices have one per 128 values (x_half_rows's e_off): a tile
+// that holds such a row (e[t] nonzero) keeps its sums in units of the current run's, rescaled
+// between the runs by powers of two.  (One exponent a row flushed what lay 2^29 below the row's
+// largest; the runs' cost 0.3 us of a launch that has none.)
 // Chunk c + DX - 1 is requested in the second half of chunk c; the one wait and barrier of a
 // chunk stand in its middle: after them chunk c + 1 is in LDS, so the last step's MFMAs run
 // with the first fragments of the next chunk on their way, and the buffer of chunk c - 1 is
@@ -31,7 +36,7 @@
 // 128 x 128 tile 60.1 (429 TFLOP/s), its four-wave form 50.9, this tile without the order 56.6,
 // with it 37.3 (690 TFLOP/s) on a ring of four chunks; 41 on five to seven, 48 on three.  Timing copies put the rest at 0.45 us
 // a chunk against 0.26 of MFMAs, plus 8 us a launch for its start, first loads and stores.
-// Seven Q8_0 products of a Qwen3-0.6B layer at M = 200: 458 -> 80 us (they had 8 to 48
+// Seven Q8_0 products of a Qwen3-0.6B layer at M = 200: 458 -> 81 us (they had 8 to 48
 // workgroups, each summing all of K).
 #include "matmul_common.h"
 
@@ -184,6 +189,10 @@ SK_DEV void matmul_ring(unsigned char *smem, const uint4 *__restrict__ w, const 
   // weight buffer of chunk c
   auto wbuf = [&](uint32_t c, uint32_t xbuf) { return TYPE == 2 ? (c >> 1) % NW : xbuf; };
 
+  // Q8_0: the rows' e[t], in the buffer that chunk DX - 1 fills after them
+  const unsigned char *const xe = xg + (DX - 1) * XB;
+  if constexpr (TYPE == 0)
+    dl_load16(masked(xres, ~0u), xg_a + (DX - 1) * XB, lane < 32 ? 4u * col0 + 16u * lane : 0x80000000u, 0);
   // ---- prologue: the first scales, chunks 0 .. DX - 2
   dma_h(s_lo, live(0));
 #pragma unroll
@@ -202,6 +211,33 @@ SK_DEV void matmul_ring(unsigned char *smem, const uint4 *__restrict__ w, const 
   for (int j = 0; j < NB; j++)
 #pragma unroll
     for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
+
+  // does a row of this tile have exponents?
+  bool big = false;
+  if constexpr (TYPE == 0) {
+    uint32_t f = lane < n_tok ? *(const uint32_t *)(xe + 4 * lane) : 0u;
+    if constexpr (NB > 2) f |= 64 + lane < n_tok ? *(const uint32_t *)(xe + 256 + 4 * lane) : 0u;
+    big = __ballot(f != 0) != 0;
+  }
+  // the sums from units of run `from` of 128 values to those of run `to` (past the last run: 1)
+  auto rescale = [&](uint32_t from, uint32_t to) {
+    const uint32_t ne = (p.n_in + E_RUN - 1) / E_RUN;
+    const int *e = (const int *)x, *er = e + p.table_off;
+    // lane l finds the change of tokens l and 64 + l, and takes its sums' from their lanes
+    int d[NB > 2 ? 2 : 1];
+#pragma unroll
+    for (int h = 0; h < (NB > 2 ? 2 : 1); h++) {
+      const uint32_t tok = 64 * h + lane, at = (col0 + tok) * ne;
+      d[h] = 0;
+      if (tok < n_tok && e[col0 + tok] != 0) d[h] = (from < ne ? er[at + from] : 0) - (to < ne ? er[at + to] : 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        acc[j][i] = __builtin_ldexpf(
+            acc[j][i], __builtin_amdgcn_ds_bpermute(4 * (4 * hh + (32 * (j & 1) + 8 * (i >> 2) + (i & 3))), d[j >> 1]));
+  };
 
   // ---- scales: hd of the current super-block; sc / nm of the next step to dequantise
   uint4 hd;
@@ -372,8 +408,10 @@ SK_DEV void matmul_ring(unsigned char *smem, const uint4 *__restrict__ w, const 
         step(IC<3>{});
         bc = bn;
       };
+      if (TYPE == 0 && __builtin_expect(big, 0)) rescale(2 * (s_lo + s) - 1, 2 * (s_lo + s));
       chunk(IC<0>{});
       chunk(IC<1>{});
+      if (TYPE == 0 && __builtin_expect(big, 0)) rescale(2 * (s_lo + s), 2 * (s_lo + s) + 1);
       chunk(IC<2>{});
       chunk(IC<3>{});
     } else if constexpr (WR > 1) {
@@ -382,6 +420,7 @@ SK_DEV void matmul_ring(unsigned char *smem, const uint4 *__restrict__ w, const 
     }
   }
   dl_wait_vm<0>();  // no load may write LDS after this
+  if (TYPE == 0 && big && n_st != 0) rescale(2 * (s_lo + n_st) - 1, ~0u);
 
   // ---- the K groups' sums.  Group wk finishes token blocks [wk NBF, wk NBF + NBF); with
   // fewer blocks than groups the first NB groups take one each.
@@ -398,9 +437,13 @@ SK_DEV void matmul_ring(unsigned char *smem, const uint4 *__restrict__ w, const 
     return tok < n_tok && row < p.n_out ? 4u * (tok * p.y_stride + row) : 0x80000000u;
   };
   float fin[NBF][16], old[ACCUM ? NBF : 1][16];
-  int4 ex[NBF][4];  // the rows came as x * 2^-e
+  int4 ex[NBF][4];  // the rows came as x * 2^-e (Q8_0: scaled back already)
 #pragma unroll
   for (int j = 0; j < NBF; j++)
+    if constexpr (TYPE == 0)
+#pragma unroll
+      for (int q = 0; q < 4; q++) ex[j][q] = make_int4(0, 0, 0, 0);
+    else
 #pragma unroll
     for (int q = 0; q < 4; q++) ex[j][q] = *(const int4 *)((const int *)x + col0 + tok0 + 32 * j + 8 * q + 4 * hh);
   if constexpr (ACCUM) {

@@ -600,15 +600,16 @@ std::vector<Command> fuse_moe(const std::vector<Command> &cmds) {
 // in by bind_workspace.  MatmulPush words: x_off 4, n_in 6, x_stride 8.
 // rows: the most input rows the launch can read (groups[0] of the prepass, rows past
 // ctl[2] x rows_per_token skip); the exponents come first, h_bytes_off bytes, then the rows.
+// e_off: where the exponents of the rows' runs of 128 values go (Q8_0 ring tile), in words.
 Launch x_half_prepass(skyla_hip_context *ctx, const Command &a, uint64_t h_bytes_off, uint32_t rows,
-                      uint32_t rows_per_token = 1) {
+                      uint32_t rows_per_token = 1, uint32_t e_off = 0) {
   Launch l;
   l.fn = ctx->x_half_rows;
   l.threads = 256;
   l.groups[0] = rows;
   l.groups[1] = l.groups[2] = 1;
   l.bufs = {a.bufs[2], nullptr, a.bufs[4]};
-  l.args = {a.push[4], a.push[8], a.push[6], (uint32_t)(h_bytes_off / 4), rows_per_token};
+  l.args = {a.push[4], a.push[8], a.push[6], (uint32_t)(h_bytes_off / 4), rows_per_token, e_off};
   l.xh_buf = 1;
   l.xh_bytes = h_bytes_off + (uint64_t)l.groups[0] * a.push[6] * 2;
   return l;
@@ -629,7 +630,8 @@ bool fusable_matmul(const Command &a, const Command &c) {
 bool ring_fits(const Command &a) {
   if (!a.ring || a.bufs[0] != a.bufs[1]) return false;
   const uint64_t rows = (uint64_t)a.groups[2] * 128, n_in = a.push[6];
-  return a.groups[0] == (a.push[7] + 127) / 128 && n_in % (a.ring->type == 0 ? 32 : 256) == 0 && rows * n_in * 2 + rows * 4 + 256 < 0x7fffffffull &&
+  return a.groups[0] == (a.push[7] + 127) / 128 && n_in % (a.ring->type == 0 ? 32 : 256) == 0 &&
+         rows * n_in * 2 + rows * 4 * (1 + (n_in + 127) / 128) + 256 < 0x7fffffffull &&
          (a.push[9] + (uint64_t)a.push[7]) * 128 * 4 < 0x7fffffffull;
 }
 
@@ -724,7 +726,7 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
         Launch f = x_half_prepass(ctx, a, h_off, rows, per_token);
         f.fn = ctx->silu_half_rows;
         f.bufs = {prev->bufs[0], nullptr, a.bufs[4]};
-        f.args = {prev->args[0], prev->args[1], a.push[8], a.push[6], (uint32_t)(h_off / 4), per_token};
+        f.args = {prev->args[0], prev->args[1], a.push[8], a.push[6], (uint32_t)(h_off / 4), per_token, 0u};
         *prev = std::move(f);
         xkey = key;
       }
@@ -800,15 +802,17 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
     const bool ring = dense && xh == "1" && ring_fits(a);
     if (ring || (dense && a.hx_fn && a.push[6] % 256 == 0)) {
       const uint32_t rows = a.groups[2] * 128;
-      const uint64_t h_off = ((uint64_t)rows * 4 + 255) & ~(uint64_t)255;
+      // Q8_0: exponents per run of 128 values after the rows' own
+      const uint32_t e_off = ring && a.ring->type == 0 ? rows : 0;
+      const uint64_t h_off = ((uint64_t)rows * 4 * (e_off ? 1 + (a.push[6] + 127) / 128 : 1) + 255) & ~(uint64_t)255;
       const std::vector<uint32_t> key = {(uint32_t)((uintptr_t)a.bufs[2] >> 32), (uint32_t)(uintptr_t)a.bufs[2],
-                                         a.push[4], a.push[8], a.push[6], a.groups[2]};
+                                         a.push[4], a.push[8], a.push[6], a.groups[2], 0u, e_off};
       if (key != xkey) {
         // The rows usually come from the launch just before: rmsnorm (q, k, v; gate and up)
         // or silu_mul (down) or the batched attention merge (o).  When it writes exactly these
         // rows, one launch does both (rmsnorm_half_rows, silu_half_rows or, for rows above 4096
         // values, silu_half_rows_wide, attention_merge_half: the same f32 and f16 rows).
-        Launch f = x_half_prepass(ctx, a, h_off, rows);
+        Launch f = x_half_prepass(ctx, a, h_off, rows, 1, e_off);
         Launch *prev = out.empty() ? nullptr : &out.back();
         const bool plain = join && prev && !prev->mark && prev->split == 0 && prev->extra.empty() && prev->xh_buf < 0 &&
                            prev->groups[2] == 1 && prev->threads == 256;
@@ -817,12 +821,13 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
             prev->groups[0] == 1 && prev->args[2] == a.push[4] && prev->args[5] == a.push[8] &&
             prev->args[3] == a.push[6] && prev->args[3] <= 4096 &&
             ((prev->args[0] | prev->args[1] | prev->args[2] | prev->args[3] | prev->args[5]) & 3u) == 0) {
-          // NormPush {x_off, w_off, y_off, n, eps, stride} + h_off; rmsnorm's grid
+          // NormPush {x_off, w_off, y_off, n, eps, stride} + {h_off, e_off}; rmsnorm's grid
           f.fn = ctx->rmsnorm_half_rows;
           f.bufs = {prev->bufs[0], prev->bufs[1], nullptr, prev->bufs[2]};
           f.xh_buf = 2;
           f.args = prev->args;
           f.args.push_back((uint32_t)(h_off / 4));
+          f.args.push_back(e_off);
           for (int d = 0; d < 3; d++) f.groups[d] = prev->groups[d];
           *prev = std::move(f);
         } else if (plain && ctx->silu_half_rows && prev->fn == ctx->silu_mul && prev->args.size() == 4 &&
@@ -832,7 +837,7 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
           // SiluPush {g_off, u_off, n, stride}, one row a token: the rows of the prepass's grid
           f.fn = ctx->silu_half_rows;
           f.bufs = {prev->bufs[0], nullptr, prev->bufs[1]};
-          f.args = {prev->args[0], prev->args[1], a.push[8], a.push[6], (uint32_t)(h_off / 4), 1u};
+          f.args = {prev->args[0], prev->args[1], a.push[8], a.push[6], (uint32_t)(h_off / 4), 1u, e_off};
           if (ctx->silu_half_wide && a.push[6] > 4096) {
             f.fn = ctx->silu_half_wide;
             f.threads = 1024;
@@ -843,13 +848,14 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
                    prev->bufs[1] == a.bufs[4] && prev->args[1] == a.push[4] && prev->args[5] == a.push[8] &&
                    prev->extra[0] <= 64 && prev->extra[0] * 128 == a.push[6] && prev->extra[1] == rows &&
                    ((prev->args[0] | prev->args[4]) & 1u) == 0) {
-          // MergePush + {n_head, h_off}; extra = {n_head, tokens} of the merge's grid
+          // MergePush + {n_head, h_off, e_off}; extra = {n_head, tokens} of the merge's grid
           f.fn = ctx->merge_half;
           f.threads = 1024;
           f.bufs = {prev->bufs[0], nullptr, prev->bufs[1]};
           f.args = prev->args;
           f.args.push_back(prev->extra[0]);
           f.args.push_back((uint32_t)(h_off / 4));
+          f.args.push_back(e_off);
           f.groups[0] = prev->extra[1];
           *prev = std::move(f);
         } else {
@@ -896,6 +902,7 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
             std::copy(c.push.begin(), c.push.end(), dst);
             dst[4] = (uint32_t)(h_off / 2);  // f16 units
             dst[8] = a.push[6];
+            dst[10] = e_off;
             start += (c.push[7] + 32 * r.wr - 1) / (32 * r.wr);
           }
         }

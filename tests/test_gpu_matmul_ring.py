@@ -5,12 +5,15 @@ rows, at the edges of their tiles.
 Bars: 3e-3 relative L2 against the oracle's f32 product (f16 operands, as the matmul tests); the
 same operands summed in another f32 order differ by at most sqrt(n_in) roundings of 2^-24 each
 way, 2 * sqrt(n_in) * 2^-24 of the result's norm.  Q8_0 without the ring converts its rows in
-the tile, in the same f16 values."""
+the tile, in the same f16 values: past f16's range, both hold each run of 128 values of a row on
+an exponent of its own."""
 import numpy as np
 import pytest
 
-from helpers import rel_l2, tactics
+from helpers import Setup, rel_l2, tactics
+from oracle import skyla_oracle as so
 from skyla_hip import engine as E
+from skyla_hip import synth
 from test_gpu_matmul import GUARD, _run
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +50,45 @@ def test_ring_shapes(ctx, dtype, n_in, n_out, n_tok, accum, split, shape):
 def test_ring_rule(ctx, dtype, n_in, n_out, n_tok):
     """The shapes the runtime's rule picks, one launch size of each of its lines."""
     _both(ctx, dtype, n_in, n_out, n_tok, True, 1)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("n_in,n_out,n_tok,split", [(1056, 140, 70, 1), (1504, 33, 200, 2), (2048, 130, 129, 4),
+                                                    (96, 64, 5, 1)])
+def test_ring_q8_range_per_run(ctx, n_in, n_out, n_tok, split, shape):
+    """A third of the tokens hold one value of 1e12 alone in its run of 128, where every weight
+    is zero (their other runs must keep their bits), a third a run of values near 1e6 or all of
+    them near 4e4, the rest none past 2^15."""
+    tag = f"{n_in}-{n_out}"
+    data = synth.matrix("mm-ring-range", tag, E.DType.Q8_0, n_in, n_out)
+    runs = -(-n_in // 128)
+    q = data.reshape(n_out, n_in // 32, 34)[:, :, 2:]
+    q[:, ::4, 5] = 0  # column 5 of every run
+    g = synth.rng("mm-ring-range", f"x-{tag}-{n_tok}")
+    x = g.standard_normal((n_tok, n_in)).astype(np.float32)
+    for t in range(n_tok):
+        r = 128 * int(g.integers(runs))
+        if t % 3 == 0:
+            x[t, r: r + 128] = 0
+            x[t, r + 5] = 1e12
+        elif t % 6 == 1:
+            x[t, r: r + 128] *= 1e6
+        elif t % 6 == 4:
+            x[t] *= 4e4
+    got = {}
+    for form in (f"{shape}_{split}", "0"):
+        with tactics(ring=form):
+            s = Setup(ctx, [(E.DType.Q8_0, n_in, n_out, data)], n_in, n_out, rows=n_tok)
+            try:
+                s.set_x(x)
+                s.matmul(0, n_tok)
+                got[form] = s.y(n_tok, n_out)
+            finally:
+                s.free()
+    want = so.matmul(int(E.DType.Q8_0), data, n_in, n_out, x)
+    for t in range(n_tok):
+        if not want[t].any():  # (a row of one run, all of it zero weights)
+            assert not got[f"{shape}_{split}"][t].any()
+            continue
+        assert rel_l2(got[f"{shape}_{split}"][t], want[t]) <= GUARD, t
+        assert rel_l2(got[f"{shape}_{split}"][t], got["0"][t]) <= 2 * np.sqrt(n_in) * 2.0 ** -24, t

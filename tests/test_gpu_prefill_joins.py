@@ -1,7 +1,8 @@
 """Prefill launches that carry the f16 row prepass of the matmul after them: the batched
 attention merge (attention_merge_half) and silu_mul in sixteen waves (silu_half_rows_wide, rows
 of more than 4096 values).  The same f32 and f16 rows as the separate launches, so the same
-logits bit for bit, over chunks with a ragged end and contexts of several splits."""
+logits bit for bit, over chunks with a ragged end and contexts of several splits, and in a Q8_0
+model whose rows pass f16's range."""
 import dataclasses
 
 import numpy as np
@@ -46,3 +47,22 @@ def test_wide_silu_with_prepass_same_logits(ctx, n_ff):
     got, n1 = _logits(ctx, c, tensors, prompt)
     want, n0 = _logits(ctx, c, tensors, prompt, xhalf_join="0")
     assert n0 > n1 and np.array_equal(got, want)
+
+
+# rows below and above the line at 4096 values
+@pytest.mark.parametrize("n_ff", [3072, 4384])
+def test_joins_past_f16_range_same_logits(ctx, n_ff):
+    """Norm weights of 1e5 put the rows that q, k, v, o, gate, up and down read past 2^15: each
+    run of 128 values then has an exponent, written by the joined launches as by x_half_rows."""
+    c = dataclasses.replace(synth.qwen3_config("tiny"), n_ff=n_ff)
+    tensors = synth.qwen3(f"{CFG}-range-{n_ff}", c, "q8_0", "random")
+    for i in range(c.n_layer):
+        for name in ("attn_norm", "ffn_norm"):
+            tensors[f"blk.{i}.{name}.weight"] = tensors[f"blk.{i}.{name}.weight"] * np.float32(1e5)
+    prompt = synth.prompt(f"{CFG}-range", E.BATCH + 22, c.n_vocab)
+    got, n1 = _logits(ctx, c, tensors, prompt)
+    want, n0 = _logits(ctx, c, tensors, prompt, xhalf_join="0", merge_join="0")
+    assert n0 > n1 and np.array_equal(got, want) and np.isfinite(got.view(np.float32)).all()
+    tile, _ = _logits(ctx, c, tensors, prompt, ring="0")
+    g, w = got.view(np.float32)[0].astype(np.float64), tile.view(np.float32)[0].astype(np.float64)
+    assert np.linalg.norm(g - w) <= 1e-2 * np.linalg.norm(w)
