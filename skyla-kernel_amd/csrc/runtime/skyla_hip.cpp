@@ -86,10 +86,12 @@ const Tactic kTactics[] = {
     {"ksnorm", "", "R_G: the Q4_K K-split form with the RMSNorm folded in on that shape"},
     {"ksglun", "1", "the norm-folded gate/up pair on its K-split form (0: LDS-staged form; R_G: shape)"},
     {"moe_fuse", "26", "bit mask of the MoE decode forms (2 gate/up pair, 8 down + combine, 16 route + pair)"},
-    {"splitk", "1", "dense K-quant matmuls of at most 128 tiles split their super-blocks (0: never)"},
+    {"splitk", "1", "dense matmuls of few tiles split their K, over launches' workgroups or (ring tiles) inside one "
+                    "(0: never)"},
     {"split_slots", "256", "workgroup slots a matmul K split fills (64..2048)"},
     {"split_stages", "2", "fewest 256-value super-blocks per split of a matmul K split (1..16)"},
-    {"seg_big", "512", "slots for a segmented matmul run past 128 tiles (gate and up at M = 128), 0: no such run"},
+    {"seg_big", "512", "slots a segmented matmul run past 128 tiles (gate and up at M = 128) fills on the 128 x 128 "
+                       "tiles (the ring tiles have their own rule); 0: no such run on either"},
     {"xhalf", "1", "f16 row prepass for matmuls on f32 rows: 1 four-wave tile where it fits, 4 without "
                    "the balanced K halves, 8 eight-wave tile throughout, 0 the tile's own f32 staging"},
     {"xhalf_moe", "1", "expert-group matmuls on f32 rows take the f16 row prepass (0: the tile's own f32 staging)"},
@@ -287,6 +289,7 @@ struct skyla_hip_pipeline {
   hipFunction_t hxm_fn = nullptr;        // expert groups (MOE = 1) on x_half_rows's f16 rows
   hipFunction_t hxms_fn = nullptr;       // and over several matrices on the same rows (segments)
   std::shared_ptr<const RingFns> ring;   // dense matmul on f16 rows: the ring tiles
+  bool k_split = true;                   // and whether they may split K (the splitk tactic)
   uint32_t split_threads = 0;
   hipFunction_t tok_fn = nullptr;        // batched form: a tok_per_wg x tok_per_wg_y block of
   uint32_t tok_per_wg = 0;               // grid.x and grid.y per workgroup
@@ -313,6 +316,7 @@ struct Command {
   hipFunction_t hx_fn = nullptr, hx4_fn = nullptr, hx4b_fn = nullptr, hxs_fn = nullptr, hxm_fn = nullptr,
                 hxms_fn = nullptr;
   std::shared_ptr<const RingFns> ring;
+  bool k_split = true;
   hipFunction_t tok_fn = nullptr;
   uint32_t tok_per_wg = 0, tok_per_wg_y = 0, tok_per_wg_z = 0, tok_threads = 0;
   std::string name;                 // the pipeline's shader name
@@ -620,7 +624,7 @@ Launch x_half_prepass(skyla_hip_context *ctx, const Command &a, uint64_t h_bytes
 // x_stride); dispatches with no barrier between them are independent.
 bool fusable_matmul(const Command &a, const Command &c) {
   return c.kind == Command::Dispatch && c.fn == a.fn && c.hx_fn == a.hx_fn && c.hxs_fn == a.hxs_fn &&
-         c.ring == a.ring && !c.segmented && c.push.size() == 13 && c.bufs == a.bufs && c.groups[1] == 1 && c.groups[2] == a.groups[2] &&
+         c.ring == a.ring && c.k_split == a.k_split && !c.segmented && c.push.size() == 13 && c.bufs == a.bufs && c.groups[1] == 1 && c.groups[2] == a.groups[2] &&
          c.push[4] == a.push[4] && c.push[6] == a.push[6] && c.push[8] == a.push[8];
 }
 
@@ -645,13 +649,13 @@ bool ring_fits(const Command &a) {
 //   fewer, short K           quarters while rows32 x token tiles x super-blocks <= 4096: 4096 x
 //                            4096 at M = 128 14.2 (26; halves split two ways 16.4), Q8_0 3072 x
 //                            1024 6.8 (43), 1024 x 3072 11.3 (126; wide 28)
-//   fewer, else              halves, split over 256 workgroups: 6144 x 4096 18.4 (25; quarters
+//   fewer, else              halves, split over 256 workgroups (split_slots): 6144 x 4096 18.4 (25; quarters
 //                            24.9), 4096 x 12288 Q4_K 28.7 (34; quarters 36), Q6_K 35.6 (40)
 // K quarters, halves and splits keep split_stages super-blocks each (Q8_0: one 256-value
 // stage); shorter rows, and every row with the splitk tactic off, are summed whole.
 int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split) {
   const uint32_t n_stage = (a.push[6] + 255) / 256;
-  const uint32_t ways = !a.split_fn && a.ring->type != 0 ? 1u : n_stage / (a.ring->type == 0 ? 1u : split_stages());
+  const uint32_t ways = a.k_split ? n_stage / (a.ring->type == 0 ? 1u : split_stages()) : 1u;
   RingShape f{};
   if (std::sscanf(tactic("ring").c_str(), "%u_%u_%u_%u_%u", &f.wr, &f.wk, &f.nb, &f.dx, split) == 5)
     for (int i = 0; i < kRingShapes; i++)
@@ -667,7 +671,7 @@ int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split
   }
   const uint64_t tok64 = (uint64_t)a.groups[2] * 2;
   if (ways >= 4 && rows32 * tok64 * n_stage <= 4096) return kRingQuarters;
-  *split = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({256 / (tiles * 2), ways / 2, 8}));
+  *split = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({split_slots() / (tiles * 2), ways / 2, 8}));
   return kRingHalves;
 }
 
@@ -1126,6 +1130,7 @@ Command dispatch_command(const skyla_hip_pipeline *p, const std::vector<void *> 
   c.hx4b_fn = p->hx4b_fn;
   c.hxs_fn = p->hxs_fn;
   c.ring = p->ring;
+  c.k_split = p->k_split;
   c.split_threads = p->split_threads;
   c.tok_fn = p->tok_fn;
   c.tok_per_wg = p->tok_per_wg;
@@ -1693,8 +1698,10 @@ int skyla_hip_pipeline_new(skyla_hip_context *ctx, const char *name, uint32_t n_
   }
   // the ring tiles of a dense matmul on f32 inputs (with the dl tactic 0: never)
   if (std::strcmp(name, "matmul") == 0 && n_spec >= 3 && spec[0] <= 2 && spec[2] == 0 && !(n_spec == 4 && spec[3]) &&
-      tactic_on("ring") && tactic_on("dl"))
+      tactic_on("ring") && tactic_on("dl")) {
     p->ring = ctx->ring[spec[0]][spec[1] & 1];
+    p->k_split = tactic_on("splitk");
+  }
   // expert-group K-quant matmul (MOE = 1) on f32 inputs: the same tile on x_half_rows's f16
   // rows (build_launches inserts the prepass of the launch's input rows)
   if (std::strcmp(name, "matmul") == 0 && n_spec >= 3 && (spec[0] == 1 || spec[0] == 2) && spec[2] == 1 &&

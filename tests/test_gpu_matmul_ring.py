@@ -92,3 +92,16 @@ def test_ring_q8_range_per_run(ctx, n_in, n_out, n_tok, split, shape):
             continue
         assert rel_l2(got[f"{shape}_{split}"][t], want[t]) <= GUARD, t
         assert rel_l2(got[f"{shape}_{split}"][t], got["0"][t]) <= 2 * np.sqrt(n_in) * 2.0 ** -24, t
+
+
+@pytest.mark.parametrize("dtype,n_in,n_out,n_tok", [(E.DType.Q8_0, 1024, 256, 60), (E.DType.Q4K, 2048, 256, 60),
+                                                    (E.DType.Q8_0, 3072, 2048, 128), (E.DType.Q6K, 4096, 4096, 128)])
+def test_ring_splitk_off_sums_whole(ctx, dtype, n_in, n_out, n_tok):
+    """Tactic splitk=0: every row in one sum, whatever the type (the bits of the unsplit wide
+    shape); by default these launches split K inside the workgroup or over several."""
+    got = {}
+    for tac in ({}, {"splitk": 0}, {"ring": "4_1_4_4_1"}):
+        with tactics(**tac):
+            got[tuple(tac)] = _run(ctx, dtype, n_in, n_out, n_tok, tag="mm-ring")[0].view(np.uint32)
+    assert np.array_equal(got["splitk",], got["ring",])
+    assert not np.array_equal(got[()], got["ring",])
