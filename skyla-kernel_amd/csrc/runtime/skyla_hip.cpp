@@ -1232,9 +1232,8 @@ const KsRule kKs3Rules[] = {{0, ~uint64_t{0}, 2, 2}};
 
 void add_ks(skyla_hip_context *ctx, const char *name, const uint32_t *spec, Retile &t) {
   const std::string ksv = tactic("ks");
-  if (ksv == "0") return;
   uint32_t fr = 0, fg = 0, fd = 0;
-  if (std::strcmp(name, "matvec_q6k") == 0 && spec[3] == 0) {
+  if (std::strcmp(name, "matvec_q6k") == 0 && spec[3] == 0 && ksv != "0") {
     // K-split Q6_K form for launches whose rows all have n_in = 12288 (matvec_q6k_ks_body):
     // three waves, RPL rows per row-group, NG row-groups per workgroup
     std::vector<KsRule> rules(std::begin(kKs6Rules), std::end(kKs6Rules));
@@ -1277,6 +1276,7 @@ void add_ks(skyla_hip_context *ctx, const char *name, const uint32_t *spec, Reti
     t.alts.insert(t.alts.end(), alts.begin(), alts.end());
     return;
   }
+  if (ksv == "0") return;
   std::string ks;
   bool pair = false, glun = false, norm = false;
   if (std::strcmp(name, "matvec_q4k") == 0 && spec[3] == 0)

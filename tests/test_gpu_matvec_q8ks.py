@@ -52,3 +52,23 @@ def test_q8_ks_forms(ctx, n_in, n_out, form, rows):
     # (y0 + product rounds once more to y0's magnitude)
     bar += 8 * 2.0 ** -24 + 2.0 ** -24 * np.linalg.norm(y0) / max(np.linalg.norm(w @ v), 1e-30)
     assert rel_l2(got, w @ v) <= bar
+
+
+def _plain(ctx, n_in, n_out, **tac):
+    data = synth.matrix("q8-ks-tactics", f"{n_in}-{n_out}", E.DType.Q8_0, n_in, n_out)
+    x = synth.activations("q8-ks-tactics", f"x-{n_in}", n_in)
+    with tactics(**tac):
+        s = Setup(ctx, [(E.DType.Q8_0, n_in, n_out, data)], n_in, n_out)
+        try:
+            s.set_x(x)
+            s.matvec(0)
+            return s.y(1, n_out)[0].view(np.uint32).copy()
+        finally:
+            s.free()
+
+
+def test_ks_off_keeps_q8_ks(ctx):
+    """Tactic ks is the K-quants': ks=0 leaves a Q8_0 launch on the form without staging."""
+    default = _plain(ctx, 3072, 500)
+    assert np.array_equal(_plain(ctx, 3072, 500, ks=0), default)
+    assert not np.array_equal(_plain(ctx, 3072, 500, q8_ks=0), default)
