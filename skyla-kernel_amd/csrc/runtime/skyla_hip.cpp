@@ -75,11 +75,11 @@ const Tactic kTactics[] = {
     {"retile", "1", "dense matvec launches take the variant the size rule gives them (0: the engine's)"},
     {"variant", "", "W_R_L: every dense launch of a matvec kernel on that (waves, rows, lanes) variant"},
     {"q8_small", "4_1_64", "W_R_L: dense Q8_0 launches (plain and SiLU-folded) below 2048 rows on that variant "
-                           "(empty: the engine's)"},
+                           "(empty: the engine's); by default those past q8_ks's n_in only"},
     {"q8_big", "4_1_16", "W_R_L: dense Q8_0 launches of 65536 rows or more (an output head) on that variant "
                          "(empty: the engine's)"},
-    {"q8_ks", "1", "Q8_0 matvecs of n_in <= 4096 below 65536 rows on the form without staging (0: never; 2, 4 or 8: "
-                   "that many rows a wave)"},
+    {"q8_ks", "1", "Q8_0 matvecs of n_in <= 4096 below 65536 rows on the form without staging, but for launches that "
+                   "a variant or q8_small entry names (0: never; 2, 4 or 8: that many rows a wave)"},
     {"ks", "1", "K-split matvec forms for n_in 4096 (Q4_K) and 12288 (Q6_K); 0: none; R_G: Q4_K shape"},
     {"ks6", "", "R_G_D: the Q6_K K-split form on that (rows, groups, groups ahead) shape"},
     {"ks3", "1", "the Q4_K K-split form for n_in 12288 (0: LDS-staged form; R_G: that shape)"},
@@ -129,6 +129,11 @@ std::string tactic(const char *key) {
     pos = end + 1;
   }
   return v;
+}
+// Does SKYLA_HIP_TACTIC hold an entry for `key`?
+bool tactic_given(const char *key) {
+  const char *env = std::getenv("SKYLA_HIP_TACTIC");
+  return env && ("," + std::string(env)).find("," + std::string(key) + "=") != std::string::npos;
 }
 bool tactic_on(const char *key) {
   const std::string v = tactic(key);
@@ -1260,6 +1265,10 @@ void add_ks(skyla_hip_context *ctx, const char *name, const uint32_t *spec, Reti
     const bool silu = std::strcmp(name, "matvec_q8_0_silu") == 0;
     if (silu && spec[1] != 1) return;
     const long forced = std::atol(tactic("q8_ks").c_str());
+    // a variant or q8_small given in the environment takes the launches it names
+    unsigned vw = 0, vr = 0, vl = 0;
+    if (std::sscanf(tactic("variant").c_str(), "%u_%u_%u", &vw, &vr, &vl) == 3) return;
+    const uint64_t from = tactic_given("q8_small") && std::strcmp(name, "matvec_q8_0_norm") != 0 ? 2048 : 0;
     std::vector<MatvecAlt> alts;
     for (uint32_t kw = 1; kw <= 4; kw++) {
       const uint32_t rw = kw == 1 ? 4 : kw == 2 ? 2 : 1;
@@ -1270,7 +1279,7 @@ void add_ks(skyla_hip_context *ctx, const char *name, const uint32_t *spec, Reti
         hipFunction_t fn = find_function(ctx, std::string(name) + "_ks__" + std::to_string(spec[1]) + "_" +
                                                   std::to_string(kw) + "_" + std::to_string(r));
         if (!fn) return;  // all or nothing
-        alts.push_back({fn, r * rw, 64 * kw * rw, q.lo, 1024 * kw, q.hi, 1024 * (kw - 1)});
+        alts.push_back({fn, r * rw, 64 * kw * rw, std::max(q.lo, from), 1024 * kw, q.hi, 1024 * (kw - 1)});
       }
     }
     t.alts.insert(t.alts.end(), alts.begin(), alts.end());

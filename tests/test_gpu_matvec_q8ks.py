@@ -72,3 +72,14 @@ def test_ks_off_keeps_q8_ks(ctx):
     default = _plain(ctx, 3072, 500)
     assert np.array_equal(_plain(ctx, 3072, 500, ks=0), default)
     assert not np.array_equal(_plain(ctx, 3072, 500, q8_ks=0), default)
+
+
+@pytest.mark.parametrize("entry,n_out,taken", [({"variant": "4_1_64"}, 500, True), ({"variant": "4_1_64"}, 3000, True),
+                                               ({"q8_small": "4_1_64"}, 500, True), ({"q8_small": ""}, 500, True),
+                                               ({"q8_small": "4_1_64"}, 2048, False)])
+def test_given_variants_act(ctx, entry, n_out, taken):
+    """A variant or q8_small entry takes the Q8_0 launches that it names from the form without
+    staging (the bits with q8_ks=0), and no others."""
+    got, staged = _plain(ctx, 3072, n_out, **entry), _plain(ctx, 3072, n_out, q8_ks=0, **entry)
+    assert np.array_equal(got, staged) == taken
+    assert np.array_equal(got, _plain(ctx, 3072, n_out)) == (not taken)
