@@ -84,10 +84,13 @@ SK_DEV int run_exp(const float4 &v) {
 // consecutive rows in a 256 B bank line and for 8 in a 128 B one
 SK_DEV uint32_t dl_swz(uint32_t r) { return (r & 7u) ^ ((r >> 3) & 1u); }
 typedef __attribute__((address_space(3))) void dl_lds;
-// vmcnt(N), the other counters unconstrained (gfx9 s_waitcnt encoding)
+// vmcnt(N), the other counters unconstrained (gfx9 s_waitcnt encoding).  The empty statement keeps
+// the reads of what the loads wrote behind the wait: where a wave reads its own loads alone no
+// barrier stands between them, and the builtin by itself claims no effect on memory.
 template <int N>
 SK_DEV void dl_wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+  asm volatile("" ::: "memory");
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
