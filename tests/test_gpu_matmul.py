@@ -111,16 +111,18 @@ def test_matmul_f16_prepass_same_bits(ctx, name, dtype, n_in, n_out, n_tok, accu
     assert rel_l2(got1, want) <= GUARD
 
 
-def test_matmul_f16_prepass_shared(ctx):
+@pytest.mark.parametrize("ring", ["1", "0"])
+def test_matmul_f16_prepass_shared(ctx, ring):
     """Two matmuls on the same rows with no barrier between them share one prepass and run as
-    one launch of two segments (two launches in all, three without the f16 rows), and each
-    gives the bits of its own f32-staged launch."""
+    one launch of two segments (two launches in all, three without the f16 rows), on the ring
+    tiles or the 128 x 128 ones, and each gives the bits of its own f32-staged launch (K in the
+    same two parts)."""
     n_in, n_tok = 1024, 70
     mats = [(E.DType.Q4K, n_in, n, synth.matrix("mm-xh", f"shared-{n}", E.DType.Q4K, n_in, n)) for n in (256, 384)]
     x = synth.activations("mm-xh", "shared-x", (n_tok, n_in))
     got = {}
     for xh in ("1", "0"):
-        with tactics(xhalf=xh):
+        with tactics(xhalf=xh, ring=ring):
             s = Setup(ctx, mats, n_in, 384, rows=2 * n_tok)
             try:
                 s.set_x(x)
@@ -155,12 +157,12 @@ CUS = 256  # MI355X: two four-wave workgroups per CU, 512 slots
     ("ragged4", E.DType.Q4K, 768, 20000, 200, True, "1"), ("ragged6", E.DType.Q6K, 768, 9000, 500, True, "1"),
 ])
 def test_matmul_balanced_grid(ctx, name, dtype, n_in, n_out, n_tok, accum, x4d):
-    """A launch of more tiles than CUs and fewer than the two-per-CU slots runs the four-wave
-    tile over a balanced grid: hf = 2 tiles - 512 tiles whole (the same bits as the plain
+    """Off the ring tiles, a launch of more tiles than CUs and fewer than the two-per-CU slots runs
+    the four-wave tile over a balanced grid: hf = 2 tiles - 512 tiles whole (the same bits as the plain
     grid, tactic xhalf=4) and the rest in two K halves added in order (within f32
     reordering of the plain grid), against the oracle at the bar; ACCUM, ragged rows and
     tokens."""
-    with tactics(dl=x4d):
+    with tactics(dl=x4d, ring=0):
         got, want = _run(ctx, dtype, n_in, n_out, n_tok, accum=accum, tag="mm-bal")
     with tactics(xhalf=4, dl=x4d):
         plain, _ = _run(ctx, dtype, n_in, n_out, n_tok, accum=accum, tag="mm-bal")
@@ -175,14 +177,15 @@ def test_matmul_balanced_grid(ctx, name, dtype, n_in, n_out, n_tok, accum, x4d):
     assert rel_l2(got, want) <= GUARD
 
 
-@pytest.mark.parametrize("dl", ["1", "0"])
+@pytest.mark.parametrize("ring,dl", [("1", "1"), ("0", "1"), ("0", "0")])
 @pytest.mark.parametrize("n_tok", [128, 100])
-def test_matmul_segments_qkv(ctx, n_tok, dl):
+def test_matmul_segments_qkv(ctx, n_tok, ring, dl):
     """q, k and v of a prefill chunk (Q4_K 4096 -> 4096, 1024, 1024 in one buffer, no barrier
     between them) run as one launch of three segments after the shared f16 row prepass: the
     bits of the three separate launches (tactic fuse=0; the same K split here: at least four
-    super-blocks a split, so four ways for all of them), and each within the bar of the
-    oracle; on the direct-to-LDS 128 x 128 tile (dl=1) and the register-staged one (dl=0)."""
+    super-blocks a split, so four parts for all of them), and each within the bar of the
+    oracle; on the ring tiles (two splits of K halves against K quarters), the direct-to-LDS
+    128 x 128 tile (ring=0) and the register-staged one (dl=0)."""
     n_in = 4096
     outs = [4096, 1024, 1024]
     mats = [(E.DType.Q4K, n_in, n, synth.matrix("mm-seg", f"qkv-{i}-{n}", E.DType.Q4K, n_in, n))
@@ -190,7 +193,7 @@ def test_matmul_segments_qkv(ctx, n_tok, dl):
     x = synth.activations("mm-seg", f"x-{n_tok}", (n_tok, n_in))
     got = {}
     for fuse in ("1", "0"):
-        with tactics(fuse=fuse, dl=dl, split_stages=4):
+        with tactics(fuse=fuse, ring=ring, dl=dl, split_stages=4):
             s = Setup(ctx, mats, n_in, max(outs), rows=len(outs) * n_tok)
             try:
                 s.set_x(x)
@@ -217,17 +220,19 @@ def test_matmul_segments_qkv(ctx, n_tok, dl):
         assert rel_l2(got["1"][1][i * n_tok:(i + 1) * n_tok, :n], want) <= GUARD
 
 
-def test_matmul_gate_up_one_launch(ctx):
+@pytest.mark.parametrize("ring", ["1", "0"])
+def test_matmul_gate_up_one_launch(ctx, ring):
     """Gate and up of a prefill chunk at M = 128 (Q4_K 4096 -> 12288 each on the same f16 rows,
-    no barrier between them: 2 x 96 row tiles) run as one launch of two segments split two
-    ways (tactic seg_big): the bits of the two separate launches (each also split two ways),
-    and within the bar of the oracle over the first 256 rows of each."""
+    no barrier between them: 2 x 96 row tiles) run as one launch of two segments (tactic
+    seg_big), on the ring tiles whole, on the 128 x 128 ones (ring=0) split two ways: the bits
+    of the two separate launches (whole, and each split two ways), and within the bar of the
+    oracle over the first 256 rows of each."""
     n_in, n_out, n_tok = 4096, 12288, 128
     mats = [(E.DType.Q4K, n_in, n_out, synth.matrix("mm-gu", f"gu-{i}", E.DType.Q4K, n_in, n_out)) for i in range(2)]
     x = synth.activations("mm-gu", f"x-{n_tok}", (n_tok, n_in))
     got = {}
     for big in ("512", "0"):
-        with tactics(seg_big=big):
+        with tactics(seg_big=big, ring=ring):
             s = Setup(ctx, mats, n_in, n_out, rows=2 * n_tok)
             try:
                 s.set_x(x)

@@ -1,6 +1,7 @@
 """The Q8_0 matvec without staging (matvec_q8_0_ks): every compiled shape (one to four waves a
 row, 2, 4 or 8 rows a wave) at the edges of its rows and columns, plain, accumulating, with the
-RMSNorm and with the SiLU folded in, against the oracle and in float64.
+RMSNorm and with the SiLU folded in, against the oracle and in float64; and the LDS-staged
+form that longer rows take (and, with q8_ks=0, these).
 
 Bar: twice the distance of a plain f32 reordering of the same product (helpers.f32_reorder_bar);
 the folded forms add the vector's own f32 roundings (a sum of squares, a division, an
@@ -18,10 +19,23 @@ pytestmark = pytest.mark.gpu
 SIZES = [(32, 1), (1024, 70), (1056, 33), (2048, 255), (2976, 13), (3072, 301), (4096, 64), (4128, 20)]
 
 
-@pytest.mark.parametrize("rows", ["1", "2", "4", "8"])
+@pytest.mark.parametrize("rows", ["0", "1", "2", "4", "8"])
 @pytest.mark.parametrize("form", [None, "accum", "norm", "silu"])
 @pytest.mark.parametrize("n_in,n_out", SIZES)
 def test_q8_ks_forms(ctx, n_in, n_out, form, rows):
+    _form(ctx, n_in, n_out, form, rows)
+
+
+# one and two staging passes of 8192 values, either side of the lines at 2048 rows and, with
+# q8_small's variant, of its four rows a workgroup
+@pytest.mark.parametrize("form", [None, "accum", "norm", "silu"])
+@pytest.mark.parametrize("n_in,n_out", [(4608, 33), (8192, 2047), (8224, 301), (12288, 1025), (4608, 2049),
+                                        (12288, 2101)])
+def test_q8_staged_rows(ctx, n_in, n_out, form):
+    _form(ctx, n_in, n_out, form, None)
+
+
+def _form(ctx, n_in, n_out, form, rows):
     g = synth.rng("q8-ks", f"{n_in}-{n_out}-{form}")
     data = synth.matrix("q8-ks", f"{n_in}-{n_out}", E.DType.Q8_0, n_in, n_out)
     x, aux = (g.standard_normal(n_in).astype(np.float32) for _ in range(2))
