@@ -645,19 +645,29 @@ bool ring_fits(const Command &a) {
 }
 
 // The ring shape and K split of a launch over `tiles` tiles of 128 rows x 128 tokens (rows32
-// blocks of 32 rows in all, n_tok tokens), from sweeps on MI355X (us, weights from HBM, the
-// eight-wave tile before it in parentheses):
-//   more than 256 tiles      two workgroups per CU: Q4_K 12288 x 4096, M = 512 65 (wide 71, 75)
-//   from 96                  wide: 24576 x 4096 at M = 128 37 (60); with 97..128 tiles half the
-//                            CUs would idle, so K in two splits: 4096 x 4096 at M = 512 31 (37),
-//                            Q6_K 4096 x 12288 83 (103)
-//   fewer, short K           quarters while rows32 x token tiles x super-blocks <= 4096: 4096 x
-//                            4096 at M = 128 14.2 (26; halves split two ways 16.4), Q8_0 3072 x
-//                            1024 6.8 (43), 1024 x 3072 11.3 (126; wide 28)
-//   fewer, else              halves, split over 256 workgroups (split_slots): 6144 x 4096 18.4 (25; quarters
-//                            24.9), 4096 x 12288 Q4_K 28.7 (34; quarters 36), Q6_K 35.6 (40)
-// K quarters, halves and splits keep split_stages super-blocks each (Q8_0: one 256-value
-// stage); shorter rows, and every row with the splitk tactic off, are summed whole.
+// blocks of 32 rows in all).  Each line with both its sides, from sweeps on MI355X (us a launch at
+// M = 128, weights from HBM; Q4_K unless said):
+//   more than 256 tiles      two workgroups per CU: n_in 4096 at 257 tiles pair 66, wide 74; at 256
+//                            tiles pair 58, wide 49
+//   129 to 256               wide: n_in 4096 at 129 tiles 37 (halves 53), at 128 37 (halves 34)
+//   43 to 128, long rows     wide, split over 256 workgroups (split_slots): n_in 12288 at 112 tiles
+//                            two ways 65 (halves 78), at 85 three ways 54 (halves 70), at 64 four
+//                            ways 44 (halves two ways 48), at 48 38 (42; Q6_K 45, 54), at 40 36
+//                            (halves three ways 36).  From 65 tiles long is past n_in 4096: 5120
+//                            at 80 30 (halves 31), 4096 at 80 26.0 (25.9), 3072 at 88 24 (22);
+//                            below, past 6144: 8192 at 64 35 (37), 5120 at 64 28 (27)
+//   fewer, K groups of few   quarters while their workgroups fill the CUs once: n_in 4096, 4096 rows
+//   stages                   (256 workgroups) 14 (halves split four ways 20), 5120 rows (320) 25
+//                            (halves, three ways 18); Q8_0 n_in 1024 at 256 8.5 (11), at 512 15
+//                            (12).  To n_in 5120 (Q8_0: 4096): 1024 rows of 4096 12.3 (13.3), of
+//                            5120 14.9 (14.7), of 6144 16.8 (15.2), of 12288 29 (19); Q8_0 of 4096
+//                            15.3 (14.9), of 5120 18.0 (16.4)
+//   fewer, else              halves, split over 256 workgroups while each of a launch's 2 S K groups
+//                            keeps three super-blocks: n_in 4096 at 64 tiles two ways 22.7, whole
+//                            24.6; n_in 2048 at 48 two ways 14.9, whole 13.4; Q8_0 n_in 1024 at 64
+//                            two ways 15.7, whole 11.4
+// K quarters and halves need split_stages super-blocks a group (Q8_0: one 256-value stage); shorter
+// rows, and every row with the splitk tactic off, are summed whole.
 int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split) {
   const uint32_t n_stage = (a.push[6] + 255) / 256;
   const uint32_t ways = a.k_split ? n_stage / (a.ring->type == 0 ? 1u : split_stages()) : 1u;
@@ -670,13 +680,15 @@ int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split
       }
   *split = 1;
   if (tiles > 256) return kRingPair;
-  if (tiles >= 96 || ways < 2) {
-    if (tiles > 96 && tiles <= 128 && ways >= 2) *split = 2;
+  if (tiles > 128 || ways < 2) return kRingWide;
+  if (tiles > 42 && n_stage > (tiles > 64 ? 16u : 24u)) {
+    *split = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(split_slots() / tiles, 8));
     return kRingWide;
   }
   const uint64_t tok64 = (uint64_t)a.groups[2] * 2;
-  if (ways >= 4 && rows32 * tok64 * n_stage <= 4096) return kRingQuarters;
-  *split = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({split_slots() / (tiles * 2), ways / 2, 8}));
+  if (ways >= 4 && rows32 * tok64 <= 256 && n_stage <= (a.ring->type == 0 ? 16u : 20u)) return kRingQuarters;
+  *split = (uint32_t)std::max<uint64_t>(
+      1, std::min<uint64_t>({split_slots() / (tiles * 2), n_stage / (2 * std::max(3u, split_stages())), 8}));
   return kRingHalves;
 }
 

@@ -224,9 +224,10 @@ def test_matmul_segments_qkv(ctx, n_tok, ring, dl):
 def test_matmul_gate_up_one_launch(ctx, ring):
     """Gate and up of a prefill chunk at M = 128 (Q4_K 4096 -> 12288 each on the same f16 rows,
     no barrier between them: 2 x 96 row tiles) run as one launch of two segments (tactic
-    seg_big), on the ring tiles whole, on the 128 x 128 ones (ring=0) split two ways: the bits
-    of the two separate launches (whole, and each split two ways), and within the bar of the
-    oracle over the first 256 rows of each."""
+    seg_big), on the 128 x 128 tiles (ring=0) split two ways with the bits of the two separate
+    launches (each also split two ways), on the ring tiles whole and within f32 reordering of
+    the separate launches (K in halves); and within the bar of the oracle over the first 256
+    rows of each."""
     n_in, n_out, n_tok = 4096, 12288, 128
     mats = [(E.DType.Q4K, n_in, n_out, synth.matrix("mm-gu", f"gu-{i}", E.DType.Q4K, n_in, n_out)) for i in range(2)]
     x = synth.activations("mm-gu", f"x-{n_tok}", (n_tok, n_in))
@@ -252,7 +253,10 @@ def test_matmul_gate_up_one_launch(ctx, ring):
             finally:
                 s.free()
     assert got["512"][0] == 2 and got["0"][0] == 3   # prepass + one launch / + two
-    assert np.array_equal(got["512"][1].view(np.uint32), got["0"][1].view(np.uint32))
+    if ring == "0":
+        assert np.array_equal(got["512"][1].view(np.uint32), got["0"][1].view(np.uint32))
+    else:
+        assert rel_l2(got["512"][1], got["0"][1]) <= 2 * np.sqrt(n_in) * 2.0 ** -24
     rows = 256
     for i, (dt, _, n, d) in enumerate(mats):
         want = so.matmul(int(dt), d[: rows * (n_in // 256) * 144], n_in, rows, x)

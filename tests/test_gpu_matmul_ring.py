@@ -45,7 +45,9 @@ def test_ring_shapes(ctx, dtype, n_in, n_out, n_tok, accum, split, shape):
 @pytest.mark.parametrize("dtype,n_in,n_out,n_tok", [
     (E.DType.Q4K, 4096, 12288, 384), (E.DType.Q4K, 4096, 12288, 128), (E.DType.Q6K, 4096, 4096, 512),
     (E.DType.Q4K, 4096, 6144, 128), (E.DType.Q4K, 4096, 4096, 100), (E.DType.Q8_0, 3072, 1024, 60),
-    (E.DType.Q8_0, 2080, 20000, 200), (E.DType.Q6K, 256, 500, 9),
+    (E.DType.Q8_0, 2080, 20000, 200), (E.DType.Q6K, 256, 500, 9), (E.DType.Q6K, 8192, 1000, 60),
+    (E.DType.Q4K, 12288, 5504, 128), (E.DType.Q6K, 6400, 8200, 100), (E.DType.Q8_0, 5120, 9000, 128),
+    (E.DType.Q8_0, 1024, 8192, 128),
 ])
 def test_ring_rule(ctx, dtype, n_in, n_out, n_tok):
     """The shapes the runtime's rule picks, one launch size of each of its lines."""
