@@ -1095,9 +1095,9 @@ extern "C" __global__ __launch_bounds__(256) void attention_merge_t__128_0(float
 // what the launch before it wrote, its time mostly the launch's own.  Measured (MI355X, merge +
 // prepass -> one launch): 128 tokens of 32 heads at positions to 512 5.2 + 4.8 -> 8.1 us, 60
 // tokens of 16 heads in one split 4.5 + 4.3 -> 4.6 us.  Bound by a head's two dependent round
-// trips (with four waves a workgroup, eight heads each, the two launches were faster).
-// Grid: one workgroup per token.
-constexpr uint32_t MHEADS = 64;
+// trips (with four waves a workgroup, eight heads each, the two launches were faster, as they are
+// with more heads or many splits: the runtime's merge_joins).  Grid: one workgroup per token.
+constexpr uint32_t MHEADS = 32;
 struct MergeHalfPush {
   MergePush m;
   uint32_t n_head, h_off, e_off;

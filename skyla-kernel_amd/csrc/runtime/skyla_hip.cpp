@@ -692,6 +692,17 @@ int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split
   return kRingHalves;
 }
 
+// Does the merge of n_head heads over a recording of n_split splits carry the next matmul's
+// prepass?  In that launch a token's heads share one workgroup of sixteen waves, so a wave merges
+// n_head / 16 of them one after another, each longer with the splits; merge and prepass as two
+// launches spread the heads over the CUs.  Two layers' chunk of 2 / 128 tokens (MI355X, us, joined
+// against separate): 16 heads, 64 splits 174 / 289 against 176 / 295, 128 splits 220 / 396 against
+// 212 / 399; 32 heads, 8 splits 168 / 235 against 168 / 237, 16 splits 173 / 263 against 166 / 264,
+// 64 splits 230 / 441 against 197 / 412; 64 heads, 2 splits 232 / 300 against 227 / 296.
+bool merge_joins(uint32_t n_head, uint32_t n_split) {
+  return n_head <= 16 ? n_split <= 64 : n_head <= 32 && n_split <= 8;
+}
+
 // The launch list of a recording.  Barriers need no command of their own: launches on one
 // stream (and the nodes of a graph captured from it) run in order.  The fuse tactic 0 keeps
 // one launch per dispatch; the xhalf tactic 0 keeps the matmuls' own f32 staging.
@@ -867,8 +878,8 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
         } else if (merge_join && ctx->merge_half && prev && !prev->mark && prev->fn == ctx->merge_t && prev->args.size() == 6 &&
                    prev->extra.size() == 2 && prev->bufs.size() == 2 && prev->bufs[0] == a.bufs[2] &&
                    prev->bufs[1] == a.bufs[4] && prev->args[1] == a.push[4] && prev->args[5] == a.push[8] &&
-                   prev->extra[0] <= 64 && prev->extra[0] * 128 == a.push[6] && prev->extra[1] == rows &&
-                   ((prev->args[0] | prev->args[4]) & 1u) == 0) {
+                   merge_joins(prev->extra[0], prev->args[2]) && prev->extra[0] * 128 == a.push[6] &&
+                   prev->extra[1] == rows && ((prev->args[0] | prev->args[4]) & 1u) == 0) {
           // MergePush + {n_head, h_off, e_off}; extra = {n_head, tokens} of the merge's grid
           f.fn = ctx->merge_half;
           f.threads = 1024;

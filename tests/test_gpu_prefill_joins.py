@@ -66,3 +66,21 @@ def test_joins_past_f16_range_same_logits(ctx, n_ff):
     tile, _ = _logits(ctx, c, tensors, prompt, ring="0")
     g, w = got.view(np.float32)[0].astype(np.float64), tile.view(np.float32)[0].astype(np.float64)
     assert np.linalg.norm(g - w) <= 1e-2 * np.linalg.norm(w)
+
+
+@pytest.mark.parametrize("n_head,n_kv,n_split,joined", [(16, 2, 64, True), (16, 2, 65, False), (32, 4, 8, True),
+                                                        (32, 4, 9, False), (40, 5, 2, False)])
+def test_merge_keeps_to_itself_past_its_heads_and_splits(ctx, n_head, n_kv, n_split, joined):
+    """The merge carries the prepass only where one workgroup a token is no slower than the two
+    launches (up to 16 heads over 64 splits, 32 over 8); elsewhere it is a launch of its own."""
+    c = dataclasses.replace(synth.qwen3_config("tiny"), n_head=n_head, n_head_kv=n_kv, n_layer=1)
+    tensors = synth.qwen3(f"{CFG}-{n_head}", c, "q4_k_m", "random")
+    n = {}
+    for join in ("1", "0"):
+        with tactics(merge_join=join):
+            eng = E.Engine(ctx, tensors, c, n_split * E.ATTENTION_CHUNK, E.KvPrecision.F16)
+            try:
+                n[join] = eng.recording(True, n_split * E.ATTENTION_CHUNK).launches()
+            finally:
+                eng.free()
+    assert n["0"] - n["1"] == (1 if joined else 0)
