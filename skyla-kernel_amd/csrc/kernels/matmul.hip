@@ -1652,9 +1652,9 @@ MMHS(1, 1)
 MMHS(2, 0)
 MMHS(2, 1)
 
-// f32 activation rows to f16 rows for the dense K-quant tiles, once per launch instead of
-// in every tile (the runtime inserts it before dense K-quant matmuls with f32 inputs; one
-// conversion serves every matmul that reads the same rows before the next barrier).  Row t
+// f32 activation rows to f16 rows for the dense tiles, once per launch instead of in every
+// tile (the runtime inserts it before dense matmuls with f32 inputs; one conversion serves
+// every matmul that reads the same rows before the next barrier).  Row t
 // (t < ctl[2]) of x -- x_off + t * x_stride, n_in values -- becomes h[t * n_in ..] =
 // f16(x * 2^-e_t), each four values k..k+3 stored in the order k, k+2, k+1, k+3 (the
 // order of the packed-quant extraction, so the tiles copy the rows as they are), with e_t = 0 unless the row's largest |x| reaches 2^15, then its

@@ -3,8 +3,9 @@
 //
 // Workgroup: WR waves over rows times WK groups of them over K; a wave owns 32 rows and all
 // 32 NB tokens of the tile, so each dequantised weight fragment feeds NB MFMAs.  K groups take
-// consecutive runs of super-blocks and their sums meet in LDS, neighbours first, as the two
-// halves of a launch split in two meet: one K partition gives the same bits in every shape.
+// consecutive runs of super-blocks and their sums meet in LDS, neighbours first; the splits of a
+// launch meet in global memory, in order.  K in two parts gives the same bits either way, and so
+// do quarters and two splits of halves; four splits add up in another order.
 //
 // Operands go from global memory straight into LDS (dl_load16), 64 k at a time:
 //   activations  f16 rows of x_half_rows, 128 B per token and chunk, 16 B units XOR-swizzled

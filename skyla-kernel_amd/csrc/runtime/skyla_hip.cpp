@@ -92,8 +92,9 @@ const Tactic kTactics[] = {
     {"split_stages", "2", "fewest 256-value super-blocks per split of a matmul K split (1..16)"},
     {"seg_big", "512", "slots a segmented matmul run past 128 tiles (gate and up at M = 128) fills on the 128 x 128 "
                        "tiles (the ring tiles have their own rule); 0: no such run on either"},
-    {"xhalf", "1", "f16 row prepass for matmuls on f32 rows: 1 four-wave tile where it fits, 4 without "
-                   "the balanced K halves, 8 eight-wave tile throughout, 0 the tile's own f32 staging"},
+    {"xhalf", "1", "f16 row prepass for matmuls on f32 rows (1: on the ring tiles, or with ring=0 on the 128 x 128 "
+                   "ones, four waves where they fit; 4: those without the balanced K halves; 8: eight waves "
+                   "throughout; 0: the tile's own f32 staging)"},
     {"xhalf_moe", "1", "expert-group matmuls on f32 rows take the f16 row prepass (0: the tile's own f32 staging)"},
     {"xhalf_join", "1", "a dense matmul's f16 row prepass runs in the rmsnorm or silu_mul launch that writes its "
                         "rows (0: a launch of its own)"},
@@ -229,7 +230,7 @@ struct skyla_hip_context {
   size_t scratch_bytes = 0;
   hipFunction_t fill_u32 = nullptr;
   uint32_t n_cu = 256;  // compute units of the device (hipDeviceProp_t.multiProcessorCount)
-  hipFunction_t x_half_rows = nullptr;  // f16 row prepass of dense K-quant matmuls (matmul.hip)
+  hipFunction_t x_half_rows = nullptr;  // f16 row prepass of dense matmuls (matmul.hip)
   hipFunction_t silu_half_rows = nullptr;  // silu_mul with the expert down projection's prepass
   hipFunction_t silu_half_wide = nullptr;  // the same in 1024 threads, for rows above 4096 values
   hipFunction_t silu_mul = nullptr;        // (moe.hip): the launch it replaces
@@ -358,9 +359,10 @@ struct Launch {
 constexpr uint32_t kMaxSeg = 4;  // MAXSEG in kernels/common.h
 constexpr uint64_t kSplitTileBytes = 128 * 128 * 4;  // one f32 partial tile (kernels/matmul.hip)
 
-// K split of a dense K-quant matmul launch (matmul.hip, matmul_tile128_w): launches of at
-// most 128 tiles of 128 x 128 leave CUs idle (the tile keeps one workgroup per CU), so
-// their super-blocks are split over up to 256 workgroups, keeping at least 4 per split.
+// K split of a dense K-quant matmul launch on the 128 x 128 tiles (matmul.hip, matmul_tile128_w;
+// the ring tiles have ring_rule): launches of at most 128 tiles leave CUs idle (the tile keeps one
+// workgroup per CU), so their super-blocks are split over up to 256 workgroups, keeping at least
+// split_stages per split.
 // Measured on MI355X at M = 512: 4096 x 4096 68.6 -> 53.0 us, 4096 x 12288 191.6 -> 119.3 us.
 // Workgroup slots a K split fills (the split_slots tactic, default 256: one eight-wave
 // workgroup per CU).
@@ -601,7 +603,7 @@ std::vector<Command> fuse_moe(const std::vector<Command> &cmds) {
   return out;
 }
 
-// f16 rows for a dense K-quant matmul with f32 inputs (matmul.hip, x_half_rows), and the
+// f16 rows for a dense matmul with f32 inputs (matmul.hip, x_half_rows), and the
 // matmul on them: the conversion the tile would do per stage, done once per launch with a
 // per-row scale, lets the tile read f16 (config-3 GEMMs 14-19% faster).  One prepass serves
 // every such matmul that reads the same rows before the next barrier (dispatches between
@@ -629,7 +631,8 @@ Launch x_half_prepass(skyla_hip_context *ctx, const Command &a, uint64_t h_bytes
 // x_stride); dispatches with no barrier between them are independent.
 bool fusable_matmul(const Command &a, const Command &c) {
   return c.kind == Command::Dispatch && c.fn == a.fn && c.hx_fn == a.hx_fn && c.hxs_fn == a.hxs_fn &&
-         c.ring == a.ring && c.k_split == a.k_split && !c.segmented && c.push.size() == 13 && c.bufs == a.bufs && c.groups[1] == 1 && c.groups[2] == a.groups[2] &&
+         c.ring == a.ring && c.k_split == a.k_split && !c.segmented && c.push.size() == 13 && c.bufs == a.bufs &&
+         c.groups[1] == 1 && c.groups[2] == a.groups[2] &&
          c.push[4] == a.push[4] && c.push[6] == a.push[6] && c.push[8] == a.push[8];
 }
 
@@ -952,6 +955,7 @@ std::vector<Launch> build_launches(skyla_hip_context *ctx, const std::vector<Com
         i += n_run;
         continue;
       }
+      // (from here: the 128 x 128 tiles, where the ring tiles do not fit or are off)
       const uint64_t max_tiles = seg_big > 0 ? 256 : 128;
       if (fuse && a.hxs_fn && a.split_fn) {
         while (n_run < kMaxSeg && i + n_run < cmds.size() && fusable_matmul(a, cmds[i + n_run]) &&
@@ -1282,9 +1286,13 @@ void add_ks(skyla_hip_context *ctx, const char *name, const uint32_t *spec, Reti
     // Q8_0 rows of at most 4096 values without staging (matvec_q8_0_ks_body): KW runs of 1024
     // values, R rows a wave by the launch's rows, so that about 256 workgroups share a launch
     // (the q8_ks tactic R forces one).  Six Qwen3-0.6B layers / a token, us: by rows 87.5 / 675,
-    // 2 everywhere 88.6 / 712, 4 88.5 / 688, 8 95.9 / 761, the LDS-staged form 110.7 / 798.  From
-    // 65536 rows (an output head) the lanes of q8_big read more bytes each than this form's
-    // activation loads cost.
+    // 2 everywhere 88.6 / 712, 4 88.5 / 688, 8 95.9 / 761, the LDS-staged form 110.7 / 798.
+    // A launch alone (us, R = 2 / 4 / 8 / LDS-staged): n_in 1024, 1024 rows 2.4 / 2.6 / 3.3 / 3.3,
+    // 8192 3.8 / 3.8 / 4.0 / 6.7, 65472 15.4 / 13.9 / 14.2 / 34.7; n_in 2048, 4096 rows 3.9 / 3.9 /
+    // 3.8 / 5.1; n_in 3072, 1024 3.1 / 2.9 / 3.2 / 4.0, 16384 13.3 / 12.2 / 11.6 / 17.8; n_in 4096,
+    // 512 2.8 / 2.9 / 3.1 / 4.1, 4096 6.3 / 5.8 / 5.5 / 7.7, 65472 60 / 51 / 46 / 76.  The lines on
+    // the rows lose up to 7% to the best R beside them.  From 65536 rows (an output head) the lanes
+    // of q8_big read more bytes each than this form's activation loads cost.
     const bool silu = std::strcmp(name, "matvec_q8_0_silu") == 0;
     if (silu && spec[1] != 1) return;
     const long forced = std::atol(tactic("q8_ks").c_str());
@@ -1715,8 +1723,9 @@ int skyla_hip_pipeline_new(skyla_hip_context *ctx, const char *name, uint32_t n_
       p->split_threads = 512;
     }
     // f32 inputs: the 128 x 128 tile on x_half_rows's f16 rows (build_launches inserts the
-    // prepass) where the ring tiles do not fit or are off, by default the forms whose operands go straight into LDS (eight waves: x8d, x8ds; four
-    // waves, Q4_K only: x4d, x4db); the dl tactic 0 keeps the register-staged tiles.
+    // prepass) where the ring tiles do not fit (ring_fits) or are off, by default the forms
+    // whose operands go straight into LDS (eight waves: x8d, x8ds; four waves, Q4_K only: x4d,
+    // x4db); the dl tactic 0 keeps the register-staged tiles.
     if (!(n_spec == 4 && spec[3])) {
       const bool dl = tactic_on("dl");
       const bool dl4 = dl && spec[0] == 1;
