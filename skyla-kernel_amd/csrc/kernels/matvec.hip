@@ -1199,17 +1199,16 @@ SK_DEV void matvec_q8_0_ks_body(const uint4 *__restrict__ w, const uint16_t *__r
     if (!live) xk[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
   if constexpr (MODE == 2) ss = wave_total(live ? ss : 0.0f);
-  // two sums of eight products a row: a lane's one product d s a row is rounded where the staged
-  // form's second is fused into its sum, and the shorter chains more than make up for it (error
-  // against 64 bits over the staged form's, n_in 32 to 4096: one chain 0.99 to 1.03, two 0.70 to 0.93)
-  const float bias0 = -128.0f * (sum4(xk[0]) + sum4(xk[1])), bias1 = -128.0f * (sum4(xk[2]) + sum4(xk[3]));
+  const float bias = -128.0f * ((sum4(xk[0]) + sum4(xk[1])) + (sum4(xk[2]) + sum4(xk[3])));
   float mine = 0.0f;
 #pragma unroll
   for (int r = 0; r < R; r++) {
-    float s = fma_bytes(q[r].x ^ SG, xk[0], bias0), s1 = fma_bytes(q[r].z ^ SG, xk[2], bias1);
+    float s = bias;
+    s = fma_bytes(q[r].x ^ SG, xk[0], s);
     s = fma_bytes(q[r].y ^ SG, xk[1], s);
-    s1 = fma_bytes(q[r].w ^ SG, xk[3], s1);
-    const float t = wave_total(live ? f16_bits_to_f32(d[r]) * (s + s1) : 0.0f);
+    s = fma_bytes(q[r].z ^ SG, xk[2], s);
+    s = fma_bytes(q[r].w ^ SG, xk[3], s);
+    const float t = wave_total(live ? f16_bits_to_f32(d[r]) * s : 0.0f);
     if (lr == (uint32_t)r) mine = t;
   }
   if constexpr (KW > 1) {
