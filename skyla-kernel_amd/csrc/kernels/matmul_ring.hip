@@ -37,7 +37,7 @@
 // 128 x 128 tile 60.1 (429 TFLOP/s), its four-wave form 50.9, this tile without the order 56.6,
 // with it 37.3 (690 TFLOP/s) on a ring of four chunks; 41 on five to seven, 48 on three.  Timing copies put the rest at 0.45 us
 // a chunk against 0.26 of MFMAs, plus 8 us a launch for its start, first loads and stores.
-// Seven Q8_0 products of a Qwen3-0.6B layer at M = 200: 458 -> 81 us (they had 8 to 48
+// Seven Q8_0 products of a Qwen3-0.6B layer at M = 200: 458 -> 75 us (they had 8 to 48
 // workgroups, each summing all of K).
 #include "matmul_common.h"
 
