@@ -662,9 +662,10 @@ bool ring_fits(const Command &a) {
 //   fewer, K groups of few   quarters while their workgroups fill the CUs once: n_in 4096, 4096 rows
 //   stages                   (256 workgroups) 14 (halves split four ways 20), 5120 rows (320) 25
 //                            (halves, three ways 18); Q8_0 n_in 1024 at 256 8.5 (11), at 512 15
-//                            (12).  To n_in 5120 (Q8_0: 4096): 1024 rows of 4096 12.3 (13.3), of
-//                            5120 14.9 (14.7), of 6144 16.8 (15.2), of 12288 29 (19); Q8_0 of 4096
-//                            15.3 (14.9), of 5120 18.0 (16.4)
+//                            (12).  To n_in 5120 (Q8_0 4096, Q6_K 6144): 1024 rows of 4096 12.3
+//                            (13.3), of 5120 14.9 (14.7), of 6144 16.8 (15.2), of 12288 29 (19);
+//                            Q8_0 of 4096 15.3 (14.9), of 5120 18.0 (16.4); Q6_K of 5120 16.3
+//                            (16.8), of 6144 18.2 (18.1), of 8192 22 (20)
 //   fewer, else              halves, split over 256 workgroups while each of a launch's 2 S K groups
 //                            keeps three super-blocks: n_in 4096 at 64 tiles two ways 22.7, whole
 //                            24.6; n_in 2048 at 48 two ways 14.9, whole 13.4; Q8_0 n_in 1024 at 64
@@ -689,7 +690,7 @@ int ring_rule(const Command &a, uint64_t tiles, uint64_t rows32, uint32_t *split
     return kRingWide;
   }
   const uint64_t tok64 = (uint64_t)a.groups[2] * 2;
-  if (ways >= 4 && rows32 * tok64 <= 256 && n_stage <= (a.ring->type == 0 ? 16u : 20u)) return kRingQuarters;
+  if (ways >= 4 && rows32 * tok64 <= 256 && n_stage <= 16 + 4 * a.ring->type) return kRingQuarters;
   *split = (uint32_t)std::max<uint64_t>(
       1, std::min<uint64_t>({split_slots() / (tiles * 2), n_stage / (2 * std::max(3u, split_stages())), 8}));
   return kRingHalves;
